@@ -217,24 +217,38 @@ hipError_t launch_gdn(const GdnArgs& a, hipStream_t stream) {
 // Three launches per segment of tokens:
 //   gdn_chunk_prep   (chunk, head, sequence): conv + SiLU, L2 norms, gates,
 //                    the two Gram matrices, the unit-triangular solve for Ut
-//                    and W (one column of [W | Ut] per thread, in registers),
-//                    and the decayed Q and K, written to a chunk record;
+//                    and W, and the decayed Q and K, written to a chunk record;
 //   gdn_chunk_state  (16-column slice of the state, head, sequence): the only
 //                    serial pass, S_{c+1} = Gamma_C S_c + Kd^T (Ut - W S_c);
-//                    it records each chunk's start state S_c and U = Ut - W S_c,
-//                    with the next chunk's W and Kd prefetched into registers
-//                    while the current one is computed;
+//                    it records each chunk's start state S_c and U = Ut - W S_c;
 //   gdn_chunk_out    (chunk, head, sequence), in parallel over the chunks:
 //                    O = Qd S_c + Aq U, then RMSNorm x norm_w x SiLU(z).
 // The state update is column-separable (column j of S only needs column j of
 // V), which is what lets the state pass split the state over 8 workgroups.
 // Every product runs on FP32 MFMA (exact FP32 products, FP32 accumulation).
+//
+// Bound at one prompt: latency.  16 heads x T/64 chunks are at most a workgroup
+// or two per CU, so each stage's time is that of its longest chain, and the
+// FP32 matrix cores (64 FLOP per clock and SIMD) set the floor of each stage.
+// The chunk record is therefore laid out as the consumers' MFMA operands (K
+// and U transposed, the state by columns, W negated): the state and output
+// passes load them from L2 straight into registers as float4, with no LDS
+// staging and no transposing stores.  T = 1000, 16 heads, one sequence, before
+// (256-thread workgroups, row-major records staged and transposed in LDS) and
+// now: prep 41.8 -> 25.8, state 52.1 -> 30.4, outputs 28.8 -> 16.3 us (125 -> 70 us per
+// layer).
 constexpr int GC_C = 64;     // tokens per chunk
 constexpr int GC_D = 128;    // key_dim = value_dim
 constexpr int GC_P = GC_D + 4;  // LDS row stride (floats) of the [C][D] tiles
+constexpr int GC_AP = GC_C + 4; // LDS row stride of [.][C] tiles
 constexpr int GC_VS = 16;    // state columns per state-pass workgroup
-// chunk record (floats): W[C][D] | Ut[C][D] (U after the state pass) | Qd[C][D] | Kd[C][D] |
-// Aq[C][C] | Gamma_C, padding | S_c[D][D] (start state, written by the state pass)
+constexpr int GC_T = 1024;   // threads of the prep kernel
+// chunk record (floats): -W[C][D] | Ut^T[D][C] (U^T after the state pass) | Qd[C][D] | Kd^T[D][C] |
+// Aq[C][C] (16x16 tiles on and below the diagonal) | Gamma_C, padding |
+// S_c^T[D][D] (start state by columns, written by the state pass).
+// Each matrix is stored as 16x16 tiles of 1 KB, row tiles outermost, a tile as
+// the float4 of its 64 lanes: lane l holds row l%16, columns 4*(l/16) .. +3 --
+// one contiguous 1 KB access per wave and MFMA operand.
 constexpr int GR_W = 0, GR_U = GC_C * GC_D, GR_Q = 2 * GC_C * GC_D, GR_K = 3 * GC_C * GC_D,
               GR_AQ = 4 * GC_C * GC_D, GR_G = GR_AQ + GC_C * GC_C, GR_S = GR_G + 64, GR_SIZE = GR_S + GC_D * GC_D;
 
@@ -246,6 +260,17 @@ constexpr int GR_W = 0, GR_U = GC_C * GC_D, GR_Q = 2 * GC_C * GC_D, GR_K = 3 * G
 __device__ __forceinline__ f32x4 mfma16(float a, float b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
+__device__ __forceinline__ f32x4 mfma16x4(f32x4 a, f32x4 b, f32x4 c) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) c = mfma16(a[q], b[q], c);
+    return c;
+}
+
+// float4 of this lane in tile (rt, ct) of a record matrix with NC column tiles
+template <int NC>
+__device__ __forceinline__ int gr_tile(int rt, int ct, int lane) { return ((rt * NC + ct) * 64 + lane) * 4; }
+__device__ __forceinline__ f32x4 ld4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+__device__ __forceinline__ void st4(float* p, f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
 
 __device__ __forceinline__ float gdn_x(const GdnArgs& a, int b, int conv_dim, int d, int tau) {
     // conv input of channel d at token tau of sequence b; tau < 0 reads the conv state
@@ -255,10 +280,28 @@ __device__ __forceinline__ float gdn_x(const GdnArgs& a, int b, int conv_dim, in
     return a.conv_state[((int64_t)b * conv_dim + d) * (a.K - 1) + (-tau - 1)];
 }
 
-__global__ __launch_bounds__(256) void gdn_chunk_prep(GdnArgs a, int t0, int nchunk, float* rec) {
-    const int c = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-    const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-    const int nh = a.nh, K = a.K;
+// Workgroups are dealt round robin to the 8 XCDs, each with its own L2: the
+// n workgroups of a (sequence, head) pair take ids of one residue mod 8, so
+// that what one of the three kernels writes for a head, and what its
+// workgroups share, stays in one L2.  Grid: 8 * n * ceil(pairs / 8).
+__device__ __forceinline__ bool gdn_pair(const GdnArgs& a, int n, int& i, int& h, int& b) {
+    const int lin = blockIdx.x, idx = lin >> 3;
+    const int pair = (lin & 7) + 8 * (idx / n);
+    i = idx % n;
+    h = pair % a.nh;
+    b = pair / a.nh;
+    return pair < a.nh * a.B;
+}
+static int gdn_grid(const GdnArgs& a, int n) { return 8 * n * ((a.nh * a.B + 7) / 8); }
+
+// One chunk of one head, 16 waves (the workgroup's LDS fills a CU, so four
+// waves per SIMD are what hides the latencies).  KT: conv taps, 0 = a.K.
+template <int KT>
+__global__ __launch_bounds__(GC_T) void gdn_chunk_prep(GdnArgs a, int t0, int nchunk, float* rec) {
+    int c, h, b;
+    if (!gdn_pair(a, nchunk, c, h, b)) return;
+    const int t = threadIdx.x, wave = t >> 6, lane = t & 63, li = lane & 15, lg = lane >> 4;
+    const int nh = a.nh, K = KT ? KT : a.K;
     const int conv_dim = 3 * nh * GC_D;
     const int tc = t0 + c * GC_C;  // first token of the chunk
 
@@ -266,95 +309,82 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep(GdnArgs a, int t0, int nch
     float* const qs = qkv_s;
     float* const ks = qkv_s + GC_C * GC_P;
     float* const vs = qkv_s + 2 * GC_C * GC_P;
-    __shared__ __attribute__((aligned(16))) float As[GC_C * GC_C];
-    __shared__ float hx[7 * 3 * GC_D];  // the K-1 inputs before the chunk: hx[j][channel] = x_{-1-j}
+    __shared__ __attribute__((aligned(16))) float As[GC_C * GC_AP];  // A^T
+    __shared__ __attribute__((aligned(16))) float Tl[4 * 256];       // inverses of A's diagonal blocks
     __shared__ double Gs[GC_C];  // decay prefix sums in FP64: their differences stay exact to ~1e-16
-    __shared__ float bs[GC_C];
+    __shared__ float bs[GC_C], gq[GC_C], gk[GC_C];  // beta_i, exp(G_i), exp(G_C - G_i)
 
-    // ---- conv1d + SiLU.  Raw inputs of the chunk go to LDS first (coalesced
-    // rows); then one thread per channel convolves in place from the last
-    // token backwards, so the inputs it still needs are not yet overwritten;
-    // the K-1 inputs before the chunk come from the rows or the conv state ----
-    {
-        // 4 consecutive channels per item, all 24 loads of a thread in flight
-        // together (vector loads when the rows allow; element loads otherwise)
+    // ---- conv1d + SiLU + L2 norms (waves 0..11): a half wave takes 8
+    // consecutive tokens of one of q, k, v, a lane 4 channels, so a token's
+    // norm is a sum over the half wave; the inputs and the K-1 before them
+    // come straight from the rows (or the conv state) into registers ----
+    if (wave < 12) {
+        constexpr int R = 8, HK = KT ? KT - 1 : 7;
+        const int hw = t >> 5, g3 = hw % 3, i0 = R * (hw / 3), ch = 4 * (t & 31);
+        const int d = g3 * nh * GC_D + h * GC_D + ch;
         const int esz = a.in_dt == DT_F32 ? 4 : 2;
+        // vector loads when the rows allow, element loads otherwise
         const bool vec = ((uintptr_t)a.mixed % (4 * esz)) == 0 && (a.ld_in % 4) == 0;
-        f32x4 xv[GC_C * 3 * GC_D / 4 / 256];
-        if (vec) {  // branch-free: rows past T are read clamped and zeroed
+        f32x4 x[R + HK];  // x[n]: token tc + i0 + n - HK
+        if (vec) {
 #pragma unroll
-            for (int v = 0; v < GC_C * 3 * GC_D / 4 / 256; ++v) {
-                const int e = t + 256 * v, i = e / (3 * GC_D / 4), cl = (e % (3 * GC_D / 4)) * 4;
-                const int d = (cl / GC_D) * nh * GC_D + h * GC_D + cl % GC_D;
-                const int tau = tc + i;
-                const int64_t o = ((int64_t)b * a.T + min(tau, a.T - 1)) * a.ld_in + d;
-                const f32x4 x = a.in_dt == DT_F32 ? *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(a.mixed) + o)
-                                                  : load_act4(a.mixed, a.in_dt, o);
-                xv[v] = tau < a.T ? x : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int n = 0; n < R + HK; ++n) {
+                if (!KT && n < HK - (K - 1)) continue;
+                const int tau = tc + i0 + n - HK;
+                const int64_t o = ((int64_t)b * a.T + max(0, min(tau, a.T - 1))) * a.ld_in + d;
+                x[n] = a.in_dt == DT_F32 ? *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(a.mixed) + o)
+                                         : load_act4(a.mixed, a.in_dt, o);
             }
         } else {
 #pragma unroll
-            for (int v = 0; v < GC_C * 3 * GC_D / 4 / 256; ++v) {
-                const int e = t + 256 * v, i = e / (3 * GC_D / 4), cl = (e % (3 * GC_D / 4)) * 4;
-                const int d = (cl / GC_D) * nh * GC_D + h * GC_D + cl % GC_D;
+            for (int n = 0; n < R + HK; ++n) {
+                if (!KT && n < HK - (K - 1)) continue;
+                const int tau = tc + i0 + n - HK;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) xv[v][q] = gdn_x(a, b, conv_dim, d + q, tc + i);
+                for (int q = 0; q < 4; ++q) x[n][q] = gdn_x(a, b, conv_dim, d + q, max(tau, 0));
             }
         }
+        if (tc + i0 < HK) {  // the sequence's first tokens: inputs before it from the conv state
 #pragma unroll
-        for (int v = 0; v < GC_C * 3 * GC_D / 4 / 256; ++v) {
-            const int e = t + 256 * v, i = e / (3 * GC_D / 4), cl = (e % (3 * GC_D / 4)) * 4;
-            const int g3 = cl / GC_D, ch = cl % GC_D;
-            *reinterpret_cast<f32x4*>(&qkv_s[g3 * GC_C * GC_P + i * GC_P + ch]) = xv[v];
-        }
-    }
-    for (int e = t; e < (K - 1) * 3 * GC_D; e += 256) {
-        const int j = e / (3 * GC_D), cl = e % (3 * GC_D), g3 = cl / GC_D, ch = cl % GC_D;
-        hx[e] = gdn_x(a, b, conv_dim, g3 * nh * GC_D + h * GC_D + ch, tc - 1 - j);
-        (void)j;
-    }
-    __syncthreads();
-    {
-        // thread = (channel, 32-token half): 384 x 2 = 3 x 256 work items; the
-        // K-1 inputs before a block are read into registers before any output
-        // is written (barrier), then each thread convolves its 32 tokens in place
-        float hist[3][7], wv[3][8];
-        int colo[3];
+            for (int n = 0; n < HK; ++n) {
+                const int tau = tc + i0 + n - HK;
+                if ((!KT && n < HK - (K - 1)) || tau >= 0) continue;
 #pragma unroll
-        for (int u = 0; u < 3; ++u) {
-            const int item = t + 256 * u, cl = item % (3 * GC_D), i0 = (item / (3 * GC_D)) * (GC_C / 2);
-            const int g3 = cl / GC_D, ch = cl % GC_D;
-            const int d = g3 * nh * GC_D + h * GC_D + ch;
-            colo[u] = g3 * GC_C * GC_P + i0 * GC_P + ch;  // offset of token i0 in qs|ks|vs
-#pragma unroll
-            for (int j = 0; j < 8; ++j) wv[u][j] = j < K ? a.conv_w[(int64_t)d * K + j] : 0.0f;
-#pragma unroll
-            for (int j = 0; j < 7; ++j) {
-                const int src = i0 - 1 - j;
-                hist[u][j] = j < K - 1 ? (src >= 0 ? qs[colo[u] - (1 + j) * GC_P] : hx[(-src - 1) * 3 * GC_D + cl]) : 0.0f;
+                for (int q = 0; q < 4; ++q) x[n][q] = gdn_x(a, b, conv_dim, d + q, tau);
             }
         }
-        __syncthreads();
+        float w[4][HK + 1];
 #pragma unroll
-        for (int u = 0; u < 3; ++u) {
-            const int item = t + 256 * u, i0 = (item / (3 * GC_D)) * (GC_C / 2);
-            const float wl = a.conv_w[(int64_t)((item % (3 * GC_D)) / GC_D * nh * GC_D + h * GC_D + item % GC_D) * K + K - 1];
-#pragma unroll 8
-            for (int i = 0; i < GC_C / 2; ++i) {
-                const float x = qs[colo[u] + i * GC_P];
-                float sum = wl * x;
+        for (int q = 0; q < 4; ++q)
 #pragma unroll
-                for (int j = 0; j < 7; ++j)
-                    if (j < K - 1) sum += wv[u][j] * hist[u][j];
+            for (int j = 0; j <= HK; ++j) w[q][j] = (KT || j < K) ? a.conv_w[(int64_t)(d + q) * K + j] : 0.0f;
+        const float qsc = g3 == 0 ? 1.0f / sqrtf((float)GC_D) : 1.0f;
 #pragma unroll
-                for (int j = 6; j > 0; --j) hist[u][j] = hist[u][j - 1];
-                hist[u][0] = x;
-                qs[colo[u] + i * GC_P] = tc + i0 + i < a.T ? silu_f(sum) : 0.0f;
+        for (int i = 0; i < R; ++i) {
+            f32x4 y;
+            float ss = 0.0f;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float wl = w[q][HK];
+                if (!KT) wl = a.conv_w[(int64_t)(d + q) * K + K - 1];
+                float sum = wl * x[i + HK][q];
+#pragma unroll
+                for (int j = 0; j < HK; ++j)
+                    if (KT || j < K - 1) sum += w[q][j] * x[i + HK - 1 - j][q];
+                y[q] = tc + i0 + i < a.T ? silu_f(sum) : 0.0f;
+                ss += y[q] * y[q];
             }
+            if (g3 < 2) {
+                ss = dpp_add<0xB1, 0xF>(ss);   // quad_perm [1,0,3,2]
+                ss = dpp_add<0x4E, 0xF>(ss);   // quad_perm [2,3,0,1]
+                ss = dpp_add<0x141, 0xF>(ss);  // row_half_mirror
+                ss = dpp_add<0x140, 0xF>(ss);  // row_mirror: every lane holds its row's sum
+                ss += __shfl_xor(ss, 16);
+                y = y * (1.0f / sqrtf(ss + 1e-6f) * qsc);
+            }
+            *reinterpret_cast<f32x4*>(&qkv_s[(g3 * GC_C + i0 + i) * GC_P + ch]) = y;
         }
-    }
-    // ---- gates and the decay prefix sum (wave 0, one token per lane) ----
-    if (wave == 0) {
+    } else if (wave == 12) {  // ---- gates and the decay prefix sum, one token per lane ----
         const int tau = tc + lane;
         double g = 0.0;
         float beta = 0.0f;
@@ -371,77 +401,60 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep(GdnArgs a, int t0, int nch
             const double o = __shfl_up(g, off);
             if (lane >= off) g += o;
         }
+        const double GC = __shfl(g, 63);
         Gs[lane] = g;
         bs[lane] = beta;
+        gq[lane] = __expf((float)g);
+        gk[lane] = __expf((float)(GC - g));
     }
     __syncthreads();
-    // ---- per-token L2 norms of q (times 1/sqrt(D)) and k: a lane pair per
-    // (token, vector), each lane summing 64 squares ----
-    {
-        const int item = t >> 1, half = t & 1;          // 128 items: token item/2, q or k
-        float* v = (item & 1 ? ks : qs) + (item >> 1) * GC_P + half * 64;
-        float ss = 0.0f;
-#pragma unroll
-        for (int d = 0; d < 64; d += 4) {
-            const float4 x = *reinterpret_cast<const float4*>(&v[d]);
-            ss += x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w;
-        }
-        ss += __shfl_xor(ss, 1);
-        const float sc = 1.0f / sqrtf(ss + 1e-6f) * (item & 1 ? 1.0f : 1.0f / sqrtf((float)GC_D));
-        __syncthreads();  // every lane has read its row
-#pragma unroll
-        for (int d = 0; d < 64; d += 4) {
-            float4 x = *reinterpret_cast<const float4*>(&v[d]);
-            x.x *= sc; x.y *= sc; x.z *= sc; x.w *= sc;
-            *reinterpret_cast<float4*>(&v[d]) = x;
-        }
-    }
-    __syncthreads();
-    // ---- Gram tiles on MFMA: the 10 lower 16x16 tiles (ti >= tj) of K K^T and
-    // Q K^T; A = beta_i exp(G_i - G_j) k_i.k_j (j < i) into LDS transposed
-    // (As[j][i]); Aq = exp(G_i - G_j) q_i.k_j (j <= i) to the record ----
+    // ---- Gram tiles on MFMA: the 10 lower 16x16 tiles (ti >= tj) of K K^T
+    // (jobs 0..9) and Q K^T (10..19); A = beta_i exp(G_i - G_j) k_i.k_j (j < i)
+    // into LDS transposed (As[j][i]); Aq = exp(G_i - G_j) q_i.k_j (j <= i) to
+    // the record (the tiles above the diagonal are never read) ----
     float* R = rec + ((int64_t)(b * nh + h) * nchunk + c) * GR_SIZE;
-    const int li = lane & 15, lg = lane >> 4;
-    for (int job = wave; job < 10; job += 4) {
-        const int ti = job < 1 ? 0 : job < 3 ? 1 : job < 6 ? 2 : 3;
-        const int tj = job - ti * (ti + 1) / 2;
-        f32x4 kk = {0.0f, 0.0f, 0.0f, 0.0f}, qk = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 2
-        for (int kb = 0; kb < GC_D; kb += 16) {
-            const f32x4 ka = *reinterpret_cast<const f32x4*>(&ks[(16 * ti + li) * GC_P + kb + 4 * lg]);
-            const f32x4 qa = *reinterpret_cast<const f32x4*>(&qs[(16 * ti + li) * GC_P + kb + 4 * lg]);
-            const f32x4 kb4 = *reinterpret_cast<const f32x4*>(&ks[(16 * tj + li) * GC_P + kb + 4 * lg]);
+    for (int job = wave; job < 20; job += 16) {
+        const int tile = job % 10;
+        const bool isq = job >= 10;
+        const int ti = tile < 1 ? 0 : tile < 3 ? 1 : tile < 6 ? 2 : 3;
+        const int tj = tile - ti * (ti + 1) / 2;
+        // K K^T gives A's tile as D[i][j]; K Q^T gives Aq's transposed, D[j][i]:
+        // a lane then holds four consecutive i of A^T's row j, and four j of Aq's row i
+        const float* xa = &ks[(16 * (isq ? tj : ti) + li) * GC_P + 4 * lg];
+        const float* xb = isq ? &qs[(16 * ti + li) * GC_P + 4 * lg] : &ks[(16 * tj + li) * GC_P + 4 * lg];
+        f32x4 g0 = {0.0f, 0.0f, 0.0f, 0.0f}, g1 = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                kk = mfma16(ka[q], kb4[q], kk);
-                qk = mfma16(qa[q], kb4[q], qk);
-            }
+        for (int kb = 0; kb < GC_D; kb += 32) {
+            g0 = mfma16x4(ld4(xa + kb), ld4(xb + kb), g0);
+            g1 = mfma16x4(ld4(xa + kb + 16), ld4(xb + kb + 16), g1);
         }
-        const int j = 16 * tj + li;
+        g0 = g0 + g1;
         f32x4 av;
+        if (isq) {
+            const int i = 16 * ti + li;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int i = 16 * ti + 4 * lg + r;
-            const float dec = j <= i ? __expf((float)(Gs[i] - Gs[j])) : 0.0f;
-            av[r] = j < i ? bs[i] * dec * kk[r] : 0.0f;
-            R[GR_AQ + i * GC_C + j] = j <= i ? dec * qk[r] : 0.0f;
+            for (int r = 0; r < 4; ++r) {
+                const int j = 16 * tj + 4 * lg + r;
+                av[r] = j <= i ? __expf((float)(Gs[i] - Gs[j])) * g0[r] : 0.0f;
+            }
+            st4(&R[GR_AQ + gr_tile<4>(ti, tj, lane)], av);
+        } else {
+            const int j = 16 * tj + li;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int i = 16 * ti + 4 * lg + r;
+                av[r] = j < i ? bs[i] * __expf((float)(Gs[i] - Gs[j])) * g0[r] : 0.0f;
+            }
+            st4(&As[j * GC_AP + 16 * ti + 4 * lg], av);
         }
-        *reinterpret_cast<f32x4*>(&As[j * GC_C + 16 * ti + 4 * lg]) = av;
-    }
-    // upper tiles of Aq are zero
-    for (int e = t; e < 6 * 256; e += 256) {
-        const int tile = e >> 8, w = e & 255;
-        const int ti = tile < 3 ? 0 : tile < 5 ? 1 : 2;
-        const int tj = ti + 1 + (tile - (ti == 0 ? 0 : ti == 1 ? 3 : 5));
-        R[GR_AQ + (16 * ti + (w >> 4)) * GC_C + 16 * tj + (w & 15)] = 0.0f;
     }
     __syncthreads();
     // ---- (I + A) X = [diag(beta Gamma) K | diag(beta) V] by 16-row blocks:
     // the four diagonal blocks are inverted by substitution (wave 0, one lane
-    // per column of a block), then each wave runs the block substitution
+    // per column of a block) while the other waves write the decayed Q and K,
+    // then each wave runs the block substitution
     //   X_b = T_bb (R_b - sum_{c<b} A_bc X_c)
-    // on MFMA for its 64 of the 256 right-hand-side columns, X in registers ----
-    __shared__ __attribute__((aligned(16))) float Tl[4 * 256];  // T_bb[m][j]
+    // on MFMA for its 16 of the 256 right-hand-side columns, X in registers ----
     if (wave == 0) {
         const int bb = lg, jc = li;
         float x[16];
@@ -449,161 +462,176 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep(GdnArgs a, int t0, int nch
         for (int m = 0; m < 16; ++m) {
             float v = m == jc ? 1.0f : 0.0f;
 #pragma unroll
-            for (int n = 0; n < m; ++n) v -= As[(16 * bb + n) * GC_C + 16 * bb + m] * x[n];
+            for (int n = 0; n < m; ++n) v -= As[(16 * bb + n) * GC_AP + 16 * bb + m] * x[n];
             x[m] = v;
         }
 #pragma unroll
         for (int m = 0; m < 16; ++m) Tl[bb * 256 + m * 16 + jc] = x[m];
+    } else {
+        for (int e = wave - 1; e < 32; e += 15) {  // 16x16 tiles (conflict-free LDS reads)
+            const int i = 16 * (e >> 3) + li, d = 16 * (e & 7) + 4 * lg;
+            st4(&R[GR_Q + (e * 64 + lane) * 4], ld4(&qs[i * GC_P + d]) * gq[i]);
+        }
+        for (int e = wave - 1; e < 32; e += 15) {
+            const int d = 16 * (e >> 2) + li, i = 16 * (e & 3) + 4 * lg;
+            f32x4 kv;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) kv[q] = ks[(i + q) * GC_P + d] * gk[i + q];
+            st4(&R[GR_K + (e * 64 + lane) * 4], kv);
+        }
     }
     __syncthreads();
     {
-        const bool isw = wave < 2;
+        const bool isw = wave < 8;
         const float* src = isw ? ks : vs;
-        const int cbase = (wave & 1) * 64;  // column base within K (waves 0, 1) or V (waves 2, 3)
-        f32x4 X[4][4];
+        const int col = (wave & 7) * 16 + li;  // column within K (waves 0..7) or V (8..15)
+        f32x4 X[4];
 #pragma unroll
         for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int i = 16 * rb + 4 * lg + r;
-                const float sc = bs[i] * (isw ? __expf((float)Gs[i]) : 1.0f);
-#pragma unroll
-                for (int ct = 0; ct < 4; ++ct) X[rb][ct][r] = sc * src[i * GC_P + cbase + 16 * ct + li];
+                X[rb][r] = bs[i] * (isw ? gq[i] : 1.0f) * src[i * GC_P + col];
             }
 #pragma unroll
         for (int rb = 0; rb < 4; ++rb) {
 #pragma unroll
             for (int cb = 0; cb < rb; ++cb) {
-                float na[4];
+                f32x4 na;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) na[q] = -As[(16 * cb + 4 * lg + q) * GC_C + 16 * rb + li];
-#pragma unroll
-                for (int ct = 0; ct < 4; ++ct)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) X[rb][ct] = mfma16(na[q], X[cb][ct][q], X[rb][ct]);
+                for (int q = 0; q < 4; ++q) na[q] = -As[(16 * cb + 4 * lg + q) * GC_AP + 16 * rb + li];
+                X[rb] = mfma16x4(na, X[cb], X[rb]);
             }
             const f32x4 ta = *reinterpret_cast<const f32x4*>(&Tl[rb * 256 + li * 16 + 4 * lg]);
+            X[rb] = mfma16x4(ta, X[rb], f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+        }
 #pragma unroll
-            for (int ct = 0; ct < 4; ++ct) {
-                f32x4 y = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int rb = 0; rb < 4; ++rb) {
+            if (isw) {  // through LDS (over q, which no wave reads any more) into row order
 #pragma unroll
-                for (int q = 0; q < 4; ++q) y = mfma16(ta[q], X[rb][ct][q], y);
-                X[rb][ct] = y;
+                for (int r = 0; r < 4; ++r) qs[(16 * rb + 4 * lg + r) * GC_P + col] = -X[rb][r];
+            } else {
+                st4(&R[GR_U + gr_tile<4>(wave & 7, rb, lane)], X[rb]);
             }
         }
-        float* dstp = R + (isw ? GR_W : GR_U) + cbase;
-#pragma unroll
-        for (int rb = 0; rb < 4; ++rb)
-#pragma unroll
-            for (int ct = 0; ct < 4; ++ct)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) dstp[(16 * rb + 4 * lg + r) * GC_D + 16 * ct + li] = X[rb][ct][r];
     }
-    // ---- decayed q and k for the scan ----
-    const double GC = Gs[GC_C - 1];
-    for (int e = t; e < GC_C * GC_D / 4; e += 256) {
-        const int i = e / (GC_D / 4), d = (e % (GC_D / 4)) * 4;
-        const float gq = __expf((float)Gs[i]), gk = __expf((float)(GC - Gs[i]));
-        float4 qv = *reinterpret_cast<const float4*>(&qs[i * GC_P + d]);
-        float4 kv = *reinterpret_cast<const float4*>(&ks[i * GC_P + d]);
-        qv.x *= gq; qv.y *= gq; qv.z *= gq; qv.w *= gq;
-        kv.x *= gk; kv.y *= gk; kv.z *= gk; kv.w *= gk;
-        *reinterpret_cast<float4*>(&R[GR_Q + i * GC_D + d]) = qv;
-        *reinterpret_cast<float4*>(&R[GR_K + i * GC_D + d]) = kv;
-    }
-    if (t == 0) R[GR_G] = __expf((float)GC);
+    __syncthreads();
+#pragma unroll
+    for (int e = wave; e < 32; e += 16)
+        st4(&R[GR_W + (e * 64 + lane) * 4], ld4(&qs[(16 * (e >> 3) + li) * GC_P + 16 * (e & 7) + 4 * lg]));
+    if (t == 0) R[GR_G] = gq[GC_C - 1];
 }
 
 // The serial pass over the chunks of one segment for a 16-column slice of
 // one head's state, on MFMA.  Per chunk: record S_c, U = Ut - W S_c (wave w:
 // rows 16w..16w+15, written over Ut), S_{c+1} = Gamma_C S_c + Kd^T U (wave w:
-// state rows 32w..32w+31).  The state slice lives in LDS transposed
-// (St[j][d]); the next chunk's W, Kd, Ut tile and Gamma_C are prefetched into
-// registers while the current one is computed.  On the last segment the
-// workgroup also moves the conv state of 48 of the head's 384 channels (the
-// prep kernel of this segment has finished reading it).
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gdn_chunk_state(GdnArgs a, int nchunk, float* rec, int last_segment) {
-    const int sl = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+// state rows 32w..32w+31, kept in registers across the chunks).  Only U and S
+// pass through LDS (12 KB); a wave's W and Kd rows are its own MFMA operands,
+// loaded two chunks ahead into two register sets, so a chunk costs its two
+// chains of 32 dependent-pair MFMAs (~0.9 us) and two barriers.  On the last
+// segment the workgroup also moves the conv state of 48 of the head's 384
+// channels (the prep kernel of this segment has finished reading it).
+__global__ __launch_bounds__(256, 2) void gdn_chunk_state(GdnArgs a, int nchunk, float* rec, int last_segment) {
+    int sl, h, b;
+    if (!gdn_pair(a, GC_D / GC_VS, sl, h, b)) return;
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63, li = lane & 15, lg = lane >> 4;
     const int nh = a.nh;
     const int c0 = sl * GC_VS;  // first state column of the slice
-    constexpr int NV = GC_C * GC_D / 4 / 256;  // float4 of W (and of Kd) per thread: 8
-    constexpr int UP = GC_C + 4;               // row stride of the transposed U tile
 
-    __shared__ __attribute__((aligned(16))) float Wl[GC_C * GC_P], Kl[GC_C * GC_P];
-    __shared__ __attribute__((aligned(16))) float St[GC_VS * GC_P], Ut[GC_VS * UP];
+    __shared__ __attribute__((aligned(16))) float St[GC_VS * GC_P], Ut[GC_VS * GC_AP];
 
-    float* Sg = a.rec_state + ((int64_t)b * nh + h) * GC_D * GC_D;
-    for (int e = t; e < GC_D * GC_VS; e += 256) {
-        const int d = e / GC_VS, j = e % GC_VS;
-        St[j * GC_P + d] = Sg[d * GC_D + c0 + j];
-    }
-
-    float* R0 = rec + (int64_t)(b * nh + h) * nchunk * GR_SIZE;
-    f32x4 wn[NV], kn[NV], un;
-    float gCn;
-    auto prefetch = [&](const float* Rc) {
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            const int e = (t + 256 * v) * 4;
-            wn[v] = *reinterpret_cast<const f32x4*>(&Rc[GR_W + e]);
-            kn[v] = *reinterpret_cast<const f32x4*>(&Rc[GR_K + e]);
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) un[r] = Rc[GR_U + (16 * wave + 4 * lg + r) * GC_D + c0 + li];
-        gCn = Rc[GR_G];
+    struct Chunk {
+        f32x4 w[8], k[2][4], u;
+        float g;
     };
-    prefetch(R0);
-    for (int c = 0; c < nchunk; ++c) {
-        float* R = R0 + (int64_t)c * GR_SIZE;
-        __syncthreads();  // the previous chunk is done with Wl, Kl, Ut; St holds S_c
+    float* R0 = rec + (int64_t)(b * nh + h) * nchunk * GR_SIZE;
+    auto load_w = [&](Chunk& x, const float* Rc) {
 #pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            const int e = (t + 256 * v) * 4, i = e / GC_D, d = e % GC_D;
-            *reinterpret_cast<f32x4*>(&Wl[i * GC_P + d]) = wn[v];
-            *reinterpret_cast<f32x4*>(&Kl[i * GC_P + d]) = kn[v];
-        }
-        f32x4 u = un;
-        const float gC = gCn;
-        if (c + 1 < nchunk) prefetch(R + GR_SIZE);  // consumed after this chunk's compute
-        // record the start state of this chunk
-        for (int e = t; e < GC_D * GC_VS; e += 256) {
-            const int d = e / GC_VS, j = e % GC_VS;
-            R[GR_S + d * GC_D + c0 + j] = St[j * GC_P + d];
-        }
-        __syncthreads();
-        // U = Ut - W S_c   (wave w: rows 16w .. 16w+15)
-#pragma unroll 4
-        for (int kb = 0; kb < GC_D; kb += 16) {
-            const f32x4 wa = *reinterpret_cast<const f32x4*>(&Wl[(16 * wave + li) * GC_P + kb + 4 * lg]);
-            const f32x4 sb = *reinterpret_cast<const f32x4*>(&St[li * GC_P + kb + 4 * lg]);
+        for (int kb = 0; kb < 8; ++kb)
+            x.w[kb] = ld4(&Rc[GR_W + gr_tile<8>(wave, kb, lane)]);
+        x.u = ld4(&Rc[GR_U + gr_tile<4>(sl, wave, lane)]);
+    };
+    auto load_k = [&](Chunk& x, const float* Rc) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) u = mfma16(-wa[q], sb[q], u);
-        }
-        *reinterpret_cast<f32x4*>(&Ut[li * UP + 16 * wave + 4 * lg]) = u;
+        for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) R[GR_U + (16 * wave + 4 * lg + r) * GC_D + c0 + li] = u[r];
-        __syncthreads();
-        // S_{c+1} = Gamma_C S_c + Kd^T U   (wave w: state rows 32w .. 32w+31)
+            for (int ib = 0; ib < 4; ++ib)
+                x.k[dt][ib] = ld4(&Rc[GR_K + gr_tile<4>(2 * wave + dt, ib, lane)]);
+        x.g = Rc[GR_G];
+    };
+    // The loads are kept in the order of their use (the scheduler would mix
+    // the two sets), so that the compiler's wait counts leave the later ones
+    // in flight.
+    Chunk x0, x1;
+    const float* R1 = R0 + (nchunk > 1 ? GR_SIZE : 0);
+    float* Sg = a.rec_state + ((int64_t)b * nh + h) * GC_D * GC_D;
+    f32x4 S[2];  // this wave's rows of the slice: S[32w + 16dt + 4lg + r][c0 + li]
 #pragma unroll
-        for (int dt = 0; dt < 2; ++dt) {
-            const int d0 = 32 * wave + 16 * dt;
-            f32x4 acc = *reinterpret_cast<const f32x4*>(&St[li * GC_P + d0 + 4 * lg]);
-            acc = acc * gC;
+    for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
-            for (int ib = 0; ib < GC_C; ib += 16) {
-                const f32x4 ub = *reinterpret_cast<const f32x4*>(&Ut[li * UP + ib + 4 * lg]);
+        for (int r = 0; r < 4; ++r) S[dt][r] = Sg[(32 * wave + 16 * dt + 4 * lg + r) * GC_D + c0 + li];
+    __builtin_amdgcn_sched_barrier(0);
+    load_w(x0, R0);
+    __builtin_amdgcn_sched_barrier(0);
+    load_k(x0, R0);
+    __builtin_amdgcn_sched_barrier(0);
+    load_w(x1, R1);
+    __builtin_amdgcn_sched_barrier(0);
+    load_k(x1, R1);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int q = 0; q < 4; ++q) acc = mfma16(Kl[(ib + 4 * lg + q) * GC_P + d0 + li], ub[q], acc);
-            }
-            *reinterpret_cast<f32x4*>(&St[li * GC_P + d0 + 4 * lg]) = acc;
-        }
-    }
+    for (int dt = 0; dt < 2; ++dt) st4(&St[li * GC_P + 32 * wave + 16 * dt + 4 * lg], S[dt]);
     __syncthreads();
-    for (int e = t; e < GC_D * GC_VS; e += 256) {
-        const int d = e / GC_VS, j = e % GC_VS;
-        Sg[d * GC_D + c0 + j] = St[j * GC_P + d];
+    auto step = [&](Chunk& x, int c) {
+        float* R = R0 + (int64_t)c * GR_SIZE;
+        const float* Rn = R0 + (int64_t)min(c + 2, nchunk - 1) * GR_SIZE;
+        // the start state of this chunk, by columns
+#pragma unroll
+        for (int dt = 0; dt < 2; ++dt)
+            st4(&R[GR_S + gr_tile<8>(sl, 2 * wave + dt, lane)], S[dt]);
+        // U = Ut - W S_c   (rows 16w .. 16w+15)
+        f32x4 u0 = x.u, u1 = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int kb = 0; kb < 8; kb += 2) {
+            u0 = mfma16x4(x.w[kb], ld4(&St[li * GC_P + 16 * kb + 4 * lg]), u0);
+            u1 = mfma16x4(x.w[kb + 1], ld4(&St[li * GC_P + 16 * kb + 16 + 4 * lg]), u1);
+        }
+        u0 = u0 + u1;
+        st4(&Ut[li * GC_AP + 16 * wave + 4 * lg], u0);
+        st4(&R[GR_U + gr_tile<4>(sl, wave, lane)], u0);
+        __builtin_amdgcn_sched_barrier(0);
+        load_w(x, Rn);
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+        // S_{c+1} = Gamma_C S_c + Kd^T U   (state rows 32w .. 32w+31)
+        S[0] = S[0] * x.g;
+        S[1] = S[1] * x.g;
+#pragma unroll
+        for (int ib = 0; ib < 4; ++ib) {
+            const f32x4 ub = ld4(&Ut[li * GC_AP + 16 * ib + 4 * lg]);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                S[0] = mfma16(x.k[0][ib][q], ub[q], S[0]);
+                S[1] = mfma16(x.k[1][ib][q], ub[q], S[1]);
+            }
+        }
+#pragma unroll
+        for (int dt = 0; dt < 2; ++dt) st4(&St[li * GC_P + 32 * wave + 16 * dt + 4 * lg], S[dt]);
+        __builtin_amdgcn_sched_barrier(0);
+        load_k(x, Rn);
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+    };
+    int c = 0;
+    for (; c + 1 < nchunk; c += 2) {
+        step(x0, c);
+        step(x1, c + 1);
     }
+    if (c < nchunk) step(x0, c);
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) Sg[(32 * wave + 16 * dt + 4 * lg + r) * GC_D + c0 + li] = S[dt][r];
 
     constexpr int CPS = 3 * GC_D / (GC_D / GC_VS);  // conv channels per slice: 48
     if (last_segment && a.K > 1 && t < CPS) {
@@ -619,103 +647,107 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     }
 }
 
-// Outputs of one chunk of one head on MFMA: O = Qd S_c + Aq U (wave w: output
-// columns 32w .. 32w+31, all 64 rows), then per token RMSNorm x norm_w x
-// SiLU(z), the row sums combined across the waves in LDS.
-__global__ __launch_bounds__(256) void gdn_chunk_out(GdnArgs a, int t0, int nchunk, const float* rec) {
-    const int c = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+// Outputs of one chunk of one head on MFMA, transposed (O^T = S^T Qd^T +
+// U^T Aq^T), so that a lane holds four consecutive output columns of a token.
+// 8 waves: wave (cg, rg) computes columns 32cg .. 32cg+31 of the token tiles rg
+// and 3 - rg (together 5 of the 10 tiles of Aq on or below the diagonal), a
+// 2 x 2 block of tiles that reads each operand tile once for two products;
+// all of a wave's S and Q tiles are in flight before its first product.
+// Then per token RMSNorm x norm_w x SiLU(z), the sums of squares combined
+// across the waves in LDS.
+__global__ __launch_bounds__(512, 2) void gdn_chunk_out(GdnArgs a, int t0, int nchunk, const float* rec) {
+    int c, h, b;
+    if (!gdn_pair(a, nchunk, c, h, b)) return;
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63, li = lane & 15, lg = lane >> 4;
-    const int nh = a.nh;
-    constexpr int AP = GC_C + 4;  // row stride of Aq and of the transposed U
-    __shared__ __attribute__((aligned(16))) float Ql[GC_C * GC_P], STl[GC_D * GC_P], Al[GC_C * AP], UTl[GC_D * AP];
+    const int cg = wave & 3, rg = wave >> 2;
+    const int rt[2] = {rg, 3 - rg};
     __shared__ float red[4][GC_C];
-    const float* R = rec + ((int64_t)(b * nh + h) * nchunk + c) * GR_SIZE;
-    for (int e = t; e < GC_C * GC_D / 4; e += 256) {
-        const int i = e / (GC_D / 4), d = (e % (GC_D / 4)) * 4;
-        *reinterpret_cast<f32x4*>(&Ql[i * GC_P + d]) = *reinterpret_cast<const f32x4*>(&R[GR_Q + i * GC_D + d]);
-        const f32x4 uv = *reinterpret_cast<const f32x4*>(&R[GR_U + i * GC_D + d]);
+    const float* R = rec + ((int64_t)(b * a.nh + h) * nchunk + c) * GR_SIZE;
+    f32x4 sa[8][2], qv[8][2];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) UTl[(d + q) * AP + i] = uv[q];
-    }
-    for (int e = t; e < GC_C * GC_C / 4; e += 256) {
-        const int i = e / (GC_C / 4), j = (e % (GC_C / 4)) * 4;
-        *reinterpret_cast<f32x4*>(&Al[i * AP + j]) = *reinterpret_cast<const f32x4*>(&R[GR_AQ + i * GC_C + j]);
-    }
-    for (int e = t; e < GC_D * GC_D / 4; e += 256) {
-        const int k = e / (GC_D / 4), j = (e % (GC_D / 4)) * 4;
-        const f32x4 sv = *reinterpret_cast<const f32x4*>(&R[GR_S + k * GC_D + j]);
+    for (int kb = 0; kb < 8; ++kb)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) STl[(j + q) * GC_P + k] = sv[q];
-    }
-    __syncthreads();
-    f32x4 o[4][2];
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-        for (int ct = 0; ct < 2; ++ct) o[rt][ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const int cb = 32 * wave;
-#pragma unroll 2
-    for (int kb = 0; kb < GC_D; kb += 16) {
-        f32x4 qa[4], sb[2];
-#pragma unroll
-        for (int rt = 0; rt < 4; ++rt) qa[rt] = *reinterpret_cast<const f32x4*>(&Ql[(16 * rt + li) * GC_P + kb + 4 * lg]);
-#pragma unroll
-        for (int ct = 0; ct < 2; ++ct) sb[ct] = *reinterpret_cast<const f32x4*>(&STl[(cb + 16 * ct + li) * GC_P + kb + 4 * lg]);
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-                for (int ct = 0; ct < 2; ++ct) o[rt][ct] = mfma16(qa[rt][q], sb[ct][q], o[rt][ct]);
-    }
-#pragma unroll
-    for (int kb = 0; kb < GC_C; kb += 16) {
-        f32x4 qa[4], sb[2];
-#pragma unroll
-        for (int rt = 0; rt < 4; ++rt) qa[rt] = *reinterpret_cast<const f32x4*>(&Al[(16 * rt + li) * AP + kb + 4 * lg]);
-#pragma unroll
-        for (int ct = 0; ct < 2; ++ct) sb[ct] = *reinterpret_cast<const f32x4*>(&UTl[(cb + 16 * ct + li) * AP + kb + 4 * lg]);
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-                for (int ct = 0; ct < 2; ++ct) o[rt][ct] = mfma16(qa[rt][q], sb[ct][q], o[rt][ct]);
-    }
-    // ---- RMSNorm x norm_w x SiLU(z) per token row: partial sums per wave ----
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            float ss = o[rt][0][r] * o[rt][0][r] + o[rt][1][r] * o[rt][1][r];
-#pragma unroll
-            for (int off = 8; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
-            if (li == 0) red[wave][16 * rt + 4 * lg + r] = ss;
+        for (int u = 0; u < 2; ++u) {
+            sa[kb][u] = ld4(&R[GR_S + gr_tile<8>(2 * cg + u, kb, lane)]);
+            qv[kb][u] = ld4(&R[GR_Q + gr_tile<8>(rt[u], kb, lane)]);
         }
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 o[2][2];  // [column tile][token tile]
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int v = 0; v < 2; ++v) o[u][v] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int kb = 0; kb < 8; ++kb)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int v = 0; v < 2; ++v) o[u][v] = mfma16(sa[kb][u][q], qv[kb][v][q], o[u][v]);
+#pragma unroll
+    for (int ib = 0; ib < 4; ++ib) {
+        if (ib > rt[1]) continue;  // uniform over the wave
+        const f32x4 u0 = ld4(&R[GR_U + gr_tile<4>(2 * cg, ib, lane)]), u1 = ld4(&R[GR_U + gr_tile<4>(2 * cg + 1, ib, lane)]);
+        const f32x4 a1 = ld4(&R[GR_AQ + gr_tile<4>(rt[1], ib, lane)]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            o[0][1] = mfma16(u0[q], a1[q], o[0][1]);
+            o[1][1] = mfma16(u1[q], a1[q], o[1][1]);
+        }
+        if (ib > rt[0]) continue;
+        const f32x4 a0 = ld4(&R[GR_AQ + gr_tile<4>(rt[0], ib, lane)]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            o[0][0] = mfma16(u0[q], a0[q], o[0][0]);
+            o[1][0] = mfma16(u1[q], a0[q], o[1][0]);
+        }
+    }
+    // ---- RMSNorm x norm_w x SiLU(z): lane (lg, li) holds columns
+    // 32cg + 16u + 4lg + r of token 16rt[v] + li in o[u][v][r] ----
+#pragma unroll
+    for (int v = 0; v < 2; ++v) {
+        float ss = 0.0f;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) ss += o[u][v][r] * o[u][v][r];
+        ss += __shfl_xor(ss, 16);
+        ss += __shfl_xor(ss, 32);
+        if (lg == 0) red[cg][16 * rt[v] + li] = ss;
+    }
+    const int esz = a.in_dt == DT_F32 ? 4 : 2, osz = a.out_dt == DT_F32 ? 4 : 2;
+    const bool zvec = ((uintptr_t)a.z % (4 * esz)) == 0 && (a.ld_in % 4) == 0;
+    const bool ovec = ((uintptr_t)a.out % (4 * osz)) == 0 && (a.ld_out % 4) == 0;
     __syncthreads();
-    const float nw0 = a.norm_w[cb + li], nw1 = a.norm_w[cb + 16 + li];
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
+    for (int v = 0; v < 2; ++v) {
+        const int i = 16 * rt[v] + li, tau = t0 + c * GC_C + i;
+        if (tau >= a.T) continue;
+        const float tot = red[0][i] + red[1][i] + red[2][i] + red[3][i];
+        const float inv = 1.0f / sqrtf(tot / (float)GC_D + 1e-6f);
+        const int64_t row = (int64_t)b * a.T + tau;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int i = 16 * rt + 4 * lg + r;
-            const int tau = t0 + c * GC_C + i;
-            if (tau >= a.T) continue;
-            const float tot = red[0][i] + red[1][i] + red[2][i] + red[3][i];
-            const float inv = 1.0f / sqrtf(tot / (float)GC_D + 1e-6f);
-            const int64_t row = (int64_t)b * a.T + tau;
-            const int64_t zi = row * a.ld_in + h * GC_D + cb + li;
-            const int64_t oi = row * a.ld_out + h * GC_D + cb + li;
-            const float y0 = o[rt][0][r] * inv * nw0 * silu_f(gdn_load(a.z, a.in_dt, zi));
-            const float y1 = o[rt][1][r] * inv * nw1 * silu_f(gdn_load(a.z, a.in_dt, zi + 16));
-            if (a.out_dt == DT_F32) {
-                reinterpret_cast<float*>(a.out)[oi] = y0;
-                reinterpret_cast<float*>(a.out)[oi + 16] = y1;
+        for (int u = 0; u < 2; ++u) {
+            const int cl = 32 * cg + 16 * u + 4 * lg;
+            const int64_t zi = row * a.ld_in + h * GC_D + cl, oi = row * a.ld_out + h * GC_D + cl;
+            f32x4 z, y;
+            if (zvec) {
+                z = load_act4(a.z, a.in_dt, zi);
             } else {
-                store_act(a.out, a.out_dt, oi, y0);
-                store_act(a.out, a.out_dt, oi + 16, y1);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) z[r] = gdn_load(a.z, a.in_dt, zi + r);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) y[r] = o[u][v][r] * inv * a.norm_w[cl + r] * silu_f(z[r]);
+            if (ovec) {
+                store_act4(a.out, a.out_dt, oi, y);
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) store_act(a.out, a.out_dt, oi + r, y[r]);
             }
         }
+    }
 }
 
 size_t gdn_chunked_bytes_per_token(int nh) { return (size_t)nh * GR_SIZE * 4 / GC_C; }
@@ -732,10 +764,13 @@ hipError_t launch_gdn_chunked(const GdnArgs& a, void* ws, size_t ws_bytes, hipSt
         const int len = (int)std::min<int64_t>(seg, a.T - t0);
         const int nchunk = (len + GC_C - 1) / GC_C;
         const bool last = t0 + len >= a.T;
-        hipLaunchKernelGGL(gdn_chunk_prep, dim3(nchunk, a.nh, a.B), dim3(256), 0, stream, a, t0, nchunk, rec);
-        hipLaunchKernelGGL(gdn_chunk_state, dim3(GC_D / GC_VS, a.nh, a.B), dim3(256), 0, stream, a, nchunk, rec,
+        if (a.K == 4)
+            hipLaunchKernelGGL(gdn_chunk_prep<4>, dim3(gdn_grid(a, nchunk)), dim3(GC_T), 0, stream, a, t0, nchunk, rec);
+        else
+            hipLaunchKernelGGL(gdn_chunk_prep<0>, dim3(gdn_grid(a, nchunk)), dim3(GC_T), 0, stream, a, t0, nchunk, rec);
+        hipLaunchKernelGGL(gdn_chunk_state, dim3(gdn_grid(a, GC_D / GC_VS)), dim3(256), 0, stream, a, nchunk, rec,
                            last ? 1 : 0);
-        hipLaunchKernelGGL(gdn_chunk_out, dim3(nchunk, a.nh, a.B), dim3(256), 0, stream, a, t0, nchunk,
+        hipLaunchKernelGGL(gdn_chunk_out, dim3(gdn_grid(a, nchunk)), dim3(512), 0, stream, a, t0, nchunk,
                            (const float*)rec);
     }
     return hipGetLastError();

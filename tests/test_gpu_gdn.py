@@ -292,3 +292,37 @@ def test_gdn_prefill_errors(qw, ctx):
         qw.gdn_prefill(ctx, P["conv_w"], P["A_log"], P["dt_bias"], P["norm_w"], x, x, x, x, cs, rs, out, NH, 4)
     with pytest.raises(qw.QwError):  # zero tokens
         qw.gdn_prefill(ctx, P["conv_w"], P["A_log"], P["dt_bias"], P["norm_w"], x, x, x, x, cs, rs, out, NH, 0)
+
+
+@pytest.mark.parametrize("T,K,io,pad", [(24, 8, "f32", 1), (65, 4, "f32", 1), (128, 5, "f16", 2), (127, 4, "bf16", 4),
+                                        (191, 4, "f32", 4)])
+def test_gdn_chunked_heads_and_strides(qw, chunk_ctx, oracle, relerr, T, K, io, pad):
+    """9 (sequence, head) pairs (a ragged deal over the 8 XCDs), run-time conv
+    taps, row strides and column offsets that forbid vector accesses (pad
+    1 and 2) or allow them (4), tokens on both sides of the 64-token chunk.
+    Bars as above; F16 outputs carry one rounding of 2^-11."""
+    nh, B = 3, 3
+    cd, vd = 3 * nh * KD, nh * VD
+    P = {k: v[:n] for (k, v), n in zip(_params(oracle, K, 990 + T).items(), (cd, nh, nh, VD))}
+    dP = {k: dev(v) for k, v in P.items()}
+    tdt = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}[io]
+    cs, rs = oracle.normal((B, cd, K - 1), 991), oracle.normal((B, nh, KD * VD), 992, 0.0, 0.3)
+    dcs, drs = dev(cs), dev(rs)
+    ld = pad + cd + vd + 2 * nh + (-(cd + vd + 2 * nh)) % 4
+    rows = dev(oracle.normal((B * T, ld), 993), tdt)
+    cut = np.cumsum([pad, cd, vd, nh, nh])
+    parts = [rows[:, i:j] for i, j in zip(cut[:-1], cut[1:])]
+    buf = torch.empty(B * T, vd + pad, device="cuda", dtype=tdt)
+    out = buf[:, pad:]
+    qw.gdn_prefill(chunk_ctx, dP["conv_w"], dP["A_log"], dP["dt_bias"], dP["norm_w"], *parts, dcs, drs, out, nh, T)
+    torch.cuda.synchronize()
+    mixed, z, a, b = (host(p).reshape(B, T, -1) for p in parts)
+    ref = np.empty((B, T, vd), np.float32)
+    for t in range(T):
+        ref[:, t], cs, rs = oracle.gdn_step(*(np.ascontiguousarray(x[:, t]) for x in (mixed, a, b, z)), P["conv_w"],
+                                            P["A_log"], P["dt_bias"], P["norm_w"], cs, rs, nh, KD, VD)
+    bar = {"f32": 2e-5, "bf16": 4e-3, "f16": 1e-3}[io]
+    got = host(out).reshape(B, T, -1)
+    assert relerr(got, ref) <= bar, relerr(got, ref)
+    assert relerr(host(drs), rs) <= 2e-5, relerr(host(drs), rs)
+    assert np.array_equal(host(dcs), cs)
