@@ -89,6 +89,7 @@ struct qw_ctx {
     int attn_vcoal = -1;         // INT8 decode V loads: -1 by launch size, 0 scattered, 1 coalesced (QW_ATTN_VCOAL)
     bool attn_fused = true;      // one-launch INT8 decode attention (QW_ATTN_FUSED=0: prep / split / combine)
     int attn_prefill_min = 16;   // tokens per sequence from which the query-block attention kernel runs (QW_ATTN_PREFILL_MIN)  // tokens per sequence from which the chunked GDN form runs (QW_GDN_CHUNK_MIN)
+    int attn_pf_min = 32;  // QW_ATTN_PF_MIN: fewest tokens per sequence of the 32-token-block INT8 prefill
     uint8_t* ws = nullptr;
     size_t ws_bytes = 0;
     // carved regions
@@ -261,6 +262,7 @@ qw_status qw_init(qw_ctx** out, int device, size_t workspace_bytes) {
     if (const char* v = getenv("QW_ATTN_SPLIT")) c->attn_split = std::max(0, atoi(v)) / 64 * 64;
     if (const char* v = getenv("QW_ATTN_VCOAL")) c->attn_vcoal = atoi(v) != 0 ? 1 : 0;
     if (const char* v = getenv("QW_ATTN_PREFILL_MIN")) c->attn_prefill_min = std::max(1, atoi(v));
+    if (const char* v = getenv("QW_ATTN_PF_MIN")) c->attn_pf_min = std::max(1, atoi(v));
     if (const char* v = getenv("QW_GDN_CHUNK_MIN")) c->gdn_chunk_min = std::max(1, atoi(v));
     if (const char* v = getenv("QW_WIDE")) c->wide = atoi(v) != 0;
     if (const char* v = getenv("QW_WIDE_MIN")) c->wide_min = std::max(1, atoi(v));
@@ -1327,6 +1329,55 @@ qw_status qw_attn_forward(qw_ctx* ctx, const qw_attn_params* p, const qw_kv_cach
         } else {
             a.split = len;
             a.nsplit = 1;
+        }
+        // INT8, longer runs: 32-token query blocks over the cache expanded to
+        // f16 MFMA operands once per segment (attn_pf), wherever the workspace
+        // holds the expanded keys and a segment of rows
+        if (cache->dtype == QW_I8 && tokens >= ctx->attn_pf_min) {
+            const int64_t keys = (std::min<int64_t>(cache->capacity, (int64_t)a.nsplit * a.split) + 63) / 64 * 64;
+            const size_t kvb = (size_t)nkv * keys * qwk::attn_pf_bytes_per_key(hd);
+            const size_t row = (size_t)nh * hd * 2, piece = qwk::attn_pf_bytes_per_piece(nh / nkv, hd);
+            int min_units = std::min(ctx->num_cus, 32);
+            // a segment of nb sequences x ntok tokens: its rows, keys and the shares of
+            // a plan for at least min_units CUs fit, and its tiles count in 31 bits
+            auto blocks = [&](int64_t n) { return (n + qwk::kPfBlock - 1) / qwk::kPfBlock; };
+            auto fits = [&](int64_t nb, int64_t ntok) {
+                return nb * (kvb + (size_t)ntok * row) + qwk::attn_pf_shares(min_units, nb * nkv * blocks(ntok)) * piece <= ws &&
+                       (double)nb * nkv * blocks(ntok) * (keys / 32 + 1) < 2147483648.0;
+            };
+            int64_t nb = 0, ntok = 0;
+            for (; ntok < 32 && min_units >= 4; min_units /= 8) {  // 32, then 4 CUs (small workspaces)
+                nb = std::min<int64_t>(batch, 65535), ntok = tokens;
+                while (nb > 1 && !fits(nb, ntok)) nb = (nb + 1) / 2;
+                while (ntok >= 32 && !fits(nb, ntok)) ntok = ntok / 2 / 32 * 32;
+            }
+            if (ntok >= 32 && keys <= (1 << 21)) {
+                for (int b0 = 0; b0 < batch; b0 += (int)nb)
+                    for (int tb = 0; tb < tokens; tb += (int)ntok) {
+                        a.b0 = b0;
+                        a.nb = (int)std::min<int64_t>(nb, batch - b0);
+                        a.tb = tb;
+                        a.ntok = (int)std::min<int64_t>(ntok, tokens - tb);
+                        a.row0 = b0 * tokens + tb;
+                        a.rows = a.nb * a.ntok;
+                        a.pf_keys = (int)keys;
+                        uint8_t* w = reinterpret_cast<uint8_t*>(ctx->xnorm) + (size_t)a.rows * row;
+                        const size_t kb = (size_t)a.nb * nkv * keys * hd * 2;
+                        a.kx = w;
+                        a.vx = w + kb;
+                        a.sx = reinterpret_cast<float*>(w + 2 * kb);
+                        a.part = a.sx + (size_t)a.nb * nkv * (keys / 32) * 128;
+                        const size_t left = ws - (size_t)a.rows * row - a.nb * kvb;
+                        const int64_t nblk = a.nb * nkv * blocks(a.ntok);
+                        a.pf_units = ctx->num_cus;
+                        while (a.pf_units > min_units && qwk::attn_pf_shares(a.pf_units, nblk) * piece > left) a.pf_units /= 2;
+                        a.pf_lone = nblk > a.pf_units || qwk::attn_pf_units(a.pf_units, nblk) * piece > left;
+                        a.pf_grid = (int)(qwk::attn_pf_units(a.pf_units, nblk) + nkv);
+                        hipError_t e = qwk::launch_attn(a, stream);
+                        if (e != hipSuccess) return hip_fail(ctx, e, "attn launch");
+                    }
+                return QW_OK;
+            }
         }
         const size_t per_row = (size_t)nh * hd * 4 + (a.nsplit > 1 ? (size_t)nh * a.nsplit * (hd + 2) * 4 : 0);
         const int64_t seq_fit = (int64_t)(ws / (per_row * (size_t)tokens));

@@ -40,17 +40,59 @@ __device__ __forceinline__ float at_load(const void* p, int dt, int64_t i) {
     return dt == DT_F32 ? reinterpret_cast<const float*>(p)[i] : load_act(p, dt, i);
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
+// E consecutive elements from i; vec: the address is a multiple of E elements
+template <int E>
+__device__ __forceinline__ void at_load_row(const void* p, int dt, int64_t i, bool vec, float (&x)[E]) {
+    if (E == 4 && vec) {
+        const f32x4 v = load_act4(p, dt, i);
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    return v;
+        for (int e = 0; e < E; ++e) x[e] = v[e];
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) x[e] = at_load(p, dt, i + e);
+}
+
+// v of lane l ^ OFF, for a value that the lanes l ^ 2 OFF, l ^ 4 OFF, .. already
+// share (a butterfly from 32 down): register moves instead of LDS round trips
+template <int OFF>
+__device__ __forceinline__ float butterfly(float v) {
+    const int x = __builtin_bit_cast(int, v);
+    if constexpr (OFF == 32 || OFF == 16) {
+        const auto s = OFF == 32 ? __builtin_amdgcn_permlane32_swap(x, x, false, false)
+                                 : __builtin_amdgcn_permlane16_swap(x, x, false, false);
+        // the two results hold both halves' values; the one that is not this lane's
+        const bool upper = threadIdx.x & OFF;
+        return __builtin_bit_cast(float, upper ? s[0] : s[1]);
+    } else {
+        // row_ror:8, row_ror:4 (= xor 4 where xor 8 agrees), quad_perm [2,3,0,1], [1,0,3,2]
+        constexpr int CTRL = OFF == 8 ? 0x128 : OFF == 4 ? 0x124 : OFF == 2 ? 0x4E : 0xB1;
+        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, x, CTRL, 0xF, 0xF, false));
+    }
+}
+
+__device__ __forceinline__ float wave_sum(float v) {
+    v += butterfly<32>(v);
+    v += butterfly<16>(v);
+    v += butterfly<8>(v);
+    v += butterfly<4>(v);
+    v += butterfly<2>(v);
+    return v + butterfly<1>(v);
 }
 
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));
-    return v;
+    v = fmaxf(v, butterfly<32>(v));
+    v = fmaxf(v, butterfly<16>(v));
+    v = fmaxf(v, butterfly<8>(v));
+    v = fmaxf(v, butterfly<4>(v));
+    v = fmaxf(v, butterfly<2>(v));
+    return fmaxf(v, butterfly<1>(v));
 }
+
+// Rotation of a pair, the roundings spelled out: every kernel that writes cache
+// codes has to round them alike.
+__device__ __forceinline__ float rope0(float x0, float x1, float c, float s) { return __builtin_fmaf(x0, c, -(x1 * s)); }
+__device__ __forceinline__ float rope1(float x0, float x1, float c, float s) { return __builtin_fmaf(x1, c, x0 * s); }
 
 // ---------------------------------------------------------------------------
 // prep: one workgroup per row with one wave per work item (nh q heads, nkv k
@@ -87,7 +129,7 @@ __global__ __launch_bounds__(1024) void attn_prep(AttnArgs a) {
         if (isq || isk) {
             float ss = 0.0f;
 #pragma unroll
-            for (int e = 0; e < E; ++e) ss += x[e] * x[e];
+            for (int e = 0; e < E; ++e) ss = __builtin_fmaf(x[e], x[e], ss);
             ss = wave_sum(ss);
             const float rms = sqrtf(ss / (float)HD + 1e-6f);
             const float* w = isq ? a.qn_w : a.kn_w;
@@ -99,8 +141,8 @@ __global__ __launch_bounds__(1024) void attn_prep(AttnArgs a) {
                 if (d < a.rot) {
                     const float c = rc[d / 2], s = rs[d / 2];
                     const float x0 = x[e], x1 = x[e + 1];
-                    x[e] = x0 * c - x1 * s;
-                    x[e + 1] = x0 * s + x1 * c;
+                    x[e] = rope0(x0, x1, c, s);
+                    x[e + 1] = rope1(x0, x1, c, s);
                 }
             }
         }
@@ -129,6 +171,125 @@ __global__ __launch_bounds__(1024) void attn_prep(AttnArgs a) {
             for (int e = 0; e < E; ++e) dst[e] = x[e];
         }
     }
+}
+
+// The same for attn_pf's segments, R rows per workgroup (the same values bit
+// for bit; q as f16).
+// The rotation's powf / cosf / sinf chain is paid once for R rows, whose loads
+// are in flight under it, and rows are read and written 16 bytes per lane: 4096
+// rows 33.6 -> 27.6 us.
+template <int HD, int R>
+__global__ __launch_bounds__(1024) void attn_prep_rows(AttnArgs a) {
+    constexpr int E = HD / 64;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    __shared__ float rc[R][HD / 2], rs[R][HD / 2];
+    const int items = a.nh + 2 * a.nkv, nr = min(R, a.rows - (int)blockIdx.x * R);
+    const int esz = a.in_dt == DT_F32 ? 4 : 2;
+    const bool vec = (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v) % (4 * esz)) == 0 && a.ld_in % 4 == 0 && a.q_hs % 4 == 0;
+    auto position = [&](int rl, int& b) {
+        const int r = a.row0 + rl;
+        b = r / a.T;
+        return a.pos[b] + r % a.T;
+    };
+    // a position outside the cache, or past the keys the launch was sized for
+    auto valid = [&](int P) { return P >= 0 && P < a.cap && P < a.nsplit * a.split; };
+    for (int it0 = 0; it0 < items; it0 += blockDim.x >> 6) {
+        const int it = it0 + wave;
+        const bool isq = it < a.nh, isk = !isq && it < a.nh + a.nkv;
+        const int h = isq ? it : (isk ? it - a.nh : it - a.nh - a.nkv);
+        const void* src = isq ? a.q : (isk ? a.k : a.v);
+        float x[R][E];
+        if (it < items) {
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                const int64_t row = (int64_t)(a.row0 + (int)blockIdx.x * R + min(i, nr - 1)) * a.ld_in;
+                const int64_t base = row + (isq ? (int64_t)h * a.q_hs : (int64_t)h * HD) + lane * E;
+                at_load_row(src, a.in_dt, base, vec, x[i]);
+            }
+        }
+        if (it0 == 0) {
+            // the rotations of these positions, shared by every q and k head
+            for (int j = threadIdx.x; j < nr * (a.rot / 2); j += blockDim.x) {
+                const int i = j / (a.rot / 2), d2 = j % (a.rot / 2);
+                int b;
+                const int P = position(blockIdx.x * R + i, b);
+                const float freq = 1.0f / powf(a.theta, (float)(2 * d2) / (float)a.rot);
+                const float ang = (float)P * freq;
+                rc[i][d2] = cosf(ang);
+                rs[i][d2] = sinf(ang);
+                if (d2 == 0 && !valid(P)) *a.err = 1u;
+            }
+            if (a.rot == 0 && (int)threadIdx.x < nr) {
+                int b;
+                if (!valid(position(blockIdx.x * R + threadIdx.x, b))) *a.err = 1u;
+            }
+            __syncthreads();
+        }
+        if (it >= items) continue;
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            if (i >= nr) break;
+            const int rl = blockIdx.x * R + i;
+            if (isq || isk) {
+                float ss = 0.0f;
+#pragma unroll
+                for (int e = 0; e < E; ++e) ss = __builtin_fmaf(x[i][e], x[i][e], ss);
+                ss = wave_sum(ss);
+                const float rms = sqrtf(ss / (float)HD + 1e-6f);
+                const float* w = isq ? a.qn_w : a.kn_w;
+#pragma unroll
+                for (int e = 0; e < E; ++e) x[i][e] = x[i][e] / rms * (1.0f + w[lane * E + e]);
+#pragma unroll
+                for (int e = 0; e < E; e += 2) {
+                    const int d = lane * E + e;
+                    if (d < a.rot) {
+                        const float c = rc[i][d / 2], s = rs[i][d / 2];
+                        const float x0 = x[i][e], x1 = x[i][e + 1];
+                        x[i][e] = rope0(x0, x1, c, s);
+                        x[i][e + 1] = rope1(x0, x1, c, s);
+                    }
+                }
+            }
+            if (isq) {
+                const int64_t qo = ((int64_t)rl * a.nh + h) * HD + lane * E;
+                typedef _Float16 f16e __attribute__((ext_vector_type(E)));
+                f16e y;
+#pragma unroll
+                for (int e = 0; e < E; ++e) y[e] = (_Float16)x[i][e];
+                *reinterpret_cast<f16e*>(reinterpret_cast<_Float16*>(a.qn) + qo) = y;
+                continue;
+            }
+            int b;
+            const int P = position(rl, b);
+            if (!valid(P)) continue;
+            const int64_t slot = ((int64_t)b * a.cap + P) * a.nkv + h;
+            float m = 0.0f;
+#pragma unroll
+            for (int e = 0; e < E; ++e) m = fmaxf(m, fabsf(x[i][e]));
+            m = wave_max(m);
+            float sc = m / 127.0f;
+            sc = sc > 1e-8f ? sc : 1.0f;
+            typedef int8_t i8e __attribute__((ext_vector_type(E)));
+            i8e y;
+#pragma unroll
+            for (int e = 0; e < E; ++e) y[e] = (int8_t)fmaxf(-127.0f, fminf(127.0f, roundf(x[i][e] / sc)));
+            int8_t* dst = reinterpret_cast<int8_t*>(isk ? a.kc : a.vc) + slot * HD + lane * E;
+            if (((uintptr_t)(isk ? a.kc : a.vc)) % E == 0) {
+                *reinterpret_cast<i8e*>(dst) = y;
+            } else {
+#pragma unroll
+                for (int e = 0; e < E; ++e) dst[e] = y[e];
+            }
+            if (lane == 0) (isk ? a.ks : a.vs)[slot] = sc;
+        }
+    }
+}
+
+template <int HD>
+static void launch_prep(const AttnArgs& a, hipStream_t stream) {
+    const dim3 t(64 * std::min(16, a.nh + 2 * a.nkv));
+    if (a.pf_units) hipLaunchKernelGGL((attn_prep_rows<HD, 4>), dim3((a.rows + 3) / 4), t, 0, stream, a);
+    else hipLaunchKernelGGL(attn_prep<HD>, dim3(a.rows), t, 0, stream, a);
 }
 
 // ---------------------------------------------------------------------------
@@ -832,6 +993,554 @@ __global__ __launch_bounds__(256) void attn_prefill_i8h(AttnArgs a) {
 }
 
 // ---------------------------------------------------------------------------
+// prefill over an INT8 cache, long token runs: three launches after the
+// segment's attn_prep.
+//
+//   attn_expand   (32-key tile, KV head, sequence): the cached codes as f16
+//                 MFMA operands, once per call instead of once per query
+//                 block: K as the A tiles of S^T = K Q^T, V^T as the A tiles of
+//                 O^T = V^T P^T, 1 KB units in the order the consumer's waves
+//                 read them, and per tile the 32 K scales (times log2(e) /
+//                 sqrt(head dim)) and the 32 V scales;
+//   attn_pf       (unit): a 64-token query block of a KV group, all its keys or,
+//                 for long blocks, a share of them;
+//   attn_pf_merge (block, 16 tokens of a head, sequence): merges the shares,
+//                 gate, output.
+//
+// Units.  A triangle of blocks has no balanced split by blocks: a block is cut
+// into n = ceil(tiles / ut) units, ut = 1.3 times the tiles per CU -- about one
+// unit per CU at 4096 tokens, no cut where the blocks alone far outnumber the
+// CUs -- and the units are dealt longest block first (1.1 times: 363 units, a
+// second round for some CUs, 142 against 118 us).  Where the blocks are
+// fewer than the CUs (pf_lone 0), uncut blocks leave a partial too: their gate
+// reads miss every cache and take 20 us in one workgroup, but are hidden by the
+// many of the merge (777 tokens: 24 instead of 42 us).  Only the device knows the
+// positions, so the plan is made there; the grid is an upper bound whose
+// superfluous workgroups come last (empty ones between the others hold up the
+// in-order dispatch: with up to 4 key splits per block in the grid, half the
+// CUs idled on average at 4096 tokens, 184 us).
+//
+// attn_pf: 2 G waves, wave (tg, w) handles the 32 tokens tg of the block for
+// query head w of the group.  Per 32-key tile: S^T (32 keys x 32 queries,
+// 32x32x16 f16 MFMA, Q in registers), online softmax per query column in FP32,
+// O^T += V^T P^T, where P^T is the score tile's own register layout (V's keys
+// are stored in that order).  Tiles reach LDS by direct loads two tiles ahead
+// (four stages), one barrier per tile.  The two waves of a SIMD belong to the
+// two token groups; group 1 runs half a tile late, so that one wave's softmax
+// runs under the other's MFMAs -- in step they take turns to idle both units.
+//
+// Bound: the f16 matrix cores (4 HD flop per key and query), closely followed
+// by the softmax's VALU work and the LDS reads of the operands (32 KB per wave
+// and tile against 1024 MFMA cycles; 16-query tiles would read twice that);
+// 64-token blocks keep the tile traffic from L2 at 256 flop per byte.
+// The running maximum is only raised when a tile exceeds it by more than a
+// factor of 2^4 (the exponentials stay below 2^4, far inside f16's range while
+// V's scales are below 1024; above, every increase counts), which leaves the
+// 128-register accumulator unscaled for nearly all tiles.  It is kept a whole
+// number (log2), so that neither it nor the cut into units changes the f16
+// rounding of the probabilities (down to f16's subnormals).
+// Measured, INT8 cache, one sequence, 4096 tokens from position 0: attn_pf 104,
+// prep 27.6, expand 5.9, merge 25.4 us (the 16-token kernels: 759, 40, -, 43); the
+// whole call 811 -> 160 us.  777 tokens: 24 + 11 + 5 + 13 us.
+constexpr int PF_Q = 64;      // tokens per query block
+constexpr int PF_KT = 32;     // keys per tile
+constexpr int PF_SC = 128;    // floats per tile of scales: 32 K | 32 V | raise threshold | padding
+constexpr int PF_MIN = 4;     // fewest tiles per unit
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ uint32_t pf_uni(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// The query blocks of one sequence, longest first: block j (tokens 64 (nblk - 1
+// - j) ..) has tiles(j) key tiles (up to two more than its last query needs).
+// The host bounds the segment's total tiles below 2^31.
+struct PfSeq {
+    uint32_t nblk, c, tmax;
+    __device__ __forceinline__ PfSeq(const AttnArgs& a, int P0) {
+        const int pend = min(a.cap, a.nsplit * a.split);
+        nblk = (a.ntok + PF_Q - 1) / PF_Q;
+        tmax = (uint32_t)(pend + PF_KT - 1) / PF_KT;
+        c = (uint32_t)(min(max(P0, 0), pend) + a.tb + PF_KT - 1) / PF_KT;
+    }
+    __device__ __forceinline__ uint32_t tiles(uint32_t j) const { return min(c + 2 * (nblk - j), tmax); }
+    __device__ __forceinline__ uint32_t all() const {  // sum over the blocks, c + 2, c + 4, .. clamped to tmax
+        const uint32_t k = tmax > c ? min((tmax - c) / 2, nblk) : 0u;  // blocks below the clamp
+        return k * c + k * (k + 1) + (nblk - k) * tmax;
+    }
+};
+
+__device__ __forceinline__ uint32_t pf_sum(uint32_t v) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    return pf_uni(v);
+}
+
+// Longest unit, in tiles, of the segment's plan.  All lanes take part.
+__device__ __forceinline__ uint32_t pf_longest(const AttnArgs& a) {
+    uint32_t v = 0;
+    for (int i = threadIdx.x & 63; i < a.nb; i += 64) v += PfSeq(a, a.pos[a.b0 + i]).all();
+    const uint32_t total = pf_sum(v) * a.nkv;
+    const uint32_t k = total / a.pf_units;
+    return max((uint32_t)PF_MIN, k + k * 3 / 10 + 2);
+}
+
+__device__ __forceinline__ uint32_t pf_shares(const PfSeq& q, uint32_t ut, uint32_t j) {
+    return max((q.tiles(j) + ut - 1) / ut, 1u);
+}
+
+// Whether a block's units leave partials
+__device__ __forceinline__ bool pf_cut(const AttnArgs& a, uint32_t n) { return n > 1 || !a.pf_lone; }
+
+// Units, and units that leave partials, of the blocks before block `end` of a
+// sequence: summed over the lanes of the wave, or by each lane for itself.
+template <bool WAVE>
+__device__ __forceinline__ void pf_count(const AttnArgs& a, const PfSeq& q, uint32_t ut, uint32_t end, uint32_t& units,
+                                         uint32_t& cut) {
+    uint32_t u = 0, k = 0;
+    for (uint32_t j = WAVE ? threadIdx.x & 63 : 0; j < end; j += WAVE ? 64 : 1) {
+        const uint32_t n = pf_shares(q, ut, j);
+        u += n;
+        k += pf_cut(a, n) ? n : 0u;
+    }
+    units = WAVE ? pf_sum(u) : u;
+    cut = WAVE ? pf_sum(k) : k;
+}
+
+// Inclusive prefix sums over the lanes of a wave.
+__device__ __forceinline__ void pf_scan(uint32_t& x, uint32_t& y) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t o = __shfl_up(x, off), k = __shfl_up(y, off);
+        if (lane >= off) {
+            x += o;
+            y += k;
+        }
+    }
+}
+
+// The sequence of unit u (of one KV head), u then relative to it, and the
+// shares of cut blocks before it; a.nb if there is none.  The lanes take
+// sequences where they outnumber the blocks, else the blocks of one after another.
+__device__ __forceinline__ int pf_seq_of(const AttnArgs& a, uint32_t ut, uint32_t& u, uint32_t& slot) {
+    const int lane = threadIdx.x & 63;
+    uint32_t units = 0, cut = 0;
+    if (a.nb == 1) return 0;
+    if (a.nb > (a.ntok + PF_Q - 1) / PF_Q) {
+        for (int i0 = 0; i0 < a.nb; i0 += 64) {
+            units = cut = 0;
+            if (i0 + lane < a.nb) {
+                const PfSeq q(a, a.pos[a.b0 + i0 + lane]);
+                pf_count<false>(a, q, ut, q.nblk, units, cut);
+            }
+            uint32_t iu = units, ic = cut;
+            pf_scan(iu, ic);
+            const uint64_t hit = __ballot(iu > u);
+            if (hit) {
+                const int first = __ffsll((unsigned long long)hit) - 1;
+                u -= pf_uni(__shfl(iu - units, first));
+                slot += pf_uni(__shfl(ic - cut, first));
+                return i0 + first;
+            }
+            u -= pf_uni(__shfl(iu, 63));
+            slot += pf_uni(__shfl(ic, 63));
+        }
+        return a.nb;
+    }
+    int bl = 0;
+    for (; bl < a.nb; ++bl) {
+        const PfSeq q(a, __builtin_amdgcn_readfirstlane(a.pos[a.b0 + bl]));
+        pf_count<true>(a, q, ut, q.nblk, units, cut);
+        if (u < units) break;
+        u -= units;
+        slot += cut;
+    }
+    return bl;
+}
+
+// floats of a share's partial: 64 rows of HD per head of the group, then (max, sum) per row
+__device__ __forceinline__ int64_t pf_piece(int G, int HD) { return (int64_t)G * PF_Q * (HD + 2); }
+
+template <int HD>
+__global__ __launch_bounds__(256) void attn_expand(AttnArgs a) {
+    constexpr int KS = HD / 16, DT = HD / 32;
+    const int tile = blockIdx.x, g = blockIdx.y, b = a.b0 + blockIdx.z;
+    const int P0 = a.pos[b];
+    const int total = min(P0 + a.tb + a.ntok, min(a.cap, a.nsplit * a.split));  // keys in the cache after attn_prep
+    const int k0 = tile * PF_KT;
+    if (P0 < 0 || k0 >= total) return;
+    const int nk = min(PF_KT, total - k0);
+    __shared__ __attribute__((aligned(16))) uint8_t Vt[PF_KT * HD];
+    const int64_t pair = (int64_t)blockIdx.z * a.nkv + g;
+    const int64_t slot0 = ((int64_t)b * a.cap + k0) * a.nkv + g;
+    const uint8_t* kbase = reinterpret_cast<const uint8_t*>(a.kc);
+    const uint8_t* vbase = reinterpret_cast<const uint8_t*>(a.vc);
+    uint8_t* kx = a.kx + (pair * a.pf_keys + k0) * (HD * 2);
+    uint8_t* vx = a.vx + (pair * a.pf_keys + k0) * (HD * 2);
+    for (int c = threadIdx.x; c < PF_KT * HD / 16; c += 256) {
+        const int key = c / (HD / 16), part = c % (HD / 16);
+        u32x4 v = {0u, 0u, 0u, 0u};
+        if (key < nk) v = *reinterpret_cast<const u32x4*>(vbase + (slot0 + (int64_t)key * a.nkv) * HD + part * 16);
+        *reinterpret_cast<u32x4*>(&Vt[key * HD + part * 16]) = v;
+    }
+    // K: unit ks, lane l: dims 16 ks + 8 (l / 32) .. +7 of key l % 32
+    for (int c = threadIdx.x; c < KS * 64; c += 256) {
+        const int ks = c >> 6, key = c & 31, hi = (c >> 5) & 1;
+        u32x2 w = {0u, 0u};
+        if (key < nk) w = *reinterpret_cast<const u32x2*>(kbase + (slot0 + (int64_t)key * a.nkv) * HD + ks * 16 + hi * 8);
+        const f16x4 x = i8x4_to_h4(w[0]), y = i8x4_to_h4(w[1]);
+        *reinterpret_cast<f16x8*>(kx + c * 16) = __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7);
+    }
+    if (threadIdx.x < 64) {
+        const int key = threadIdx.x & 31;
+        const bool isv = threadIdx.x >= 32;
+        float v = key < nk ? (isv ? a.vs : a.ks)[slot0 + (int64_t)key * a.nkv] : 0.0f;
+        // the V scales' maximum decides how far the running maximum may lag
+        float big = isv ? v : 0.0f;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) big = fmaxf(big, __shfl_xor(big, off));
+        if (!isv) v *= 1.44269504f / sqrtf((float)HD);
+        float* sx = a.sx + (pair * (a.pf_keys / PF_KT) + tile) * PF_SC;
+        sx[threadIdx.x] = v;
+        if (threadIdx.x == 0) sx[64] = big < 1024.0f ? 4.0f : 0.0f;
+    }
+    __syncthreads();
+    // V: unit (m, dt), lane l: dim 32 dt + l % 32 of the keys that lane half
+    // l / 32 holds of a score tile's rows 16 m .. 16 m + 15
+    for (int c = threadIdx.x; c < 2 * DT * 64; c += 256) {
+        const int m = c / (DT * 64), d = (c >> 6) % DT * 32 + (c & 31), hi = (c >> 5) & 1;
+        f16x8 o;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int key = 16 * m + 4 * hi + (j & 3) + 8 * (j >> 2);
+            o[j] = (_Float16)(short)(int8_t)Vt[key * HD + d];
+        }
+        *reinterpret_cast<f16x8*>(vx + c * 16) = o;
+    }
+}
+
+template <int HD>
+__global__ __launch_bounds__(512, 2) void attn_pf(AttnArgs a) {
+    constexpr int KS = HD / 16, DT = HD / 32, LA = 3;
+    constexpr int KB = PF_KT * HD * 2;      // bytes of a K (or V) tile: 16 KB
+    constexpr int ST = 2 * KB + 512, NS = 4;  // a stage: K | V | scales
+    static_assert(8 * 16 * HD * 4 <= NS * ST, "output rows over the stages");
+    __shared__ __attribute__((aligned(16))) uint8_t lds[NS * ST];
+
+    const int G = a.nh / a.nkv;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, li = lane & 31, hi = lane >> 5;
+    const int tg = wave >= G, w = wave - tg * G;
+    // unit -> (sequence, KV head, block, share); the KV heads take turns, so that
+    // with two of them an XCD (workgroup ids mod 8) reads the keys of one
+    const uint32_t ut = pf_longest(a);
+    uint32_t u = blockIdx.x / a.nkv, slot = 0;
+    const int g = blockIdx.x % a.nkv;
+    const int bl = pf_seq_of(a, ut, u, slot);
+    if (bl >= a.nb) return;  // uniform
+    const int P0 = __builtin_amdgcn_readfirstlane(a.pos[a.b0 + bl]);
+    const PfSeq sq(a, P0);
+    uint32_t jb = 0, n = 0;  // block in unit order, its units; u: the share
+    for (uint32_t j0 = 0; j0 < sq.nblk; j0 += 64) {
+        const uint32_t v = j0 + lane < sq.nblk ? pf_shares(sq, ut, j0 + lane) : 0u, k = pf_cut(a, v) ? v : 0u;
+        uint32_t iu = v, ic = k;
+        pf_scan(iu, ic);
+        const uint64_t hit = __ballot(iu > u);
+        if (hit) {
+            const int first = __ffsll((unsigned long long)hit) - 1;
+            n = pf_uni(__shfl(v, first));
+            jb = j0 + first;
+            u -= pf_uni(__shfl(iu - v, first));
+            slot += pf_uni(__shfl(ic - k, first)) + u;
+            break;
+        }
+        u -= pf_uni(__shfl(iu, 63));
+        slot += pf_uni(__shfl(ic, 63));
+    }
+    if (n == 0) return;  // past the last unit; uniform
+    const int qb = (int)(sq.nblk - 1 - jb);
+    const int pend = min(a.cap, a.nsplit * a.split);
+    const int b = a.b0 + bl, h = g * G + w, tok0 = a.tb + qb * PF_Q + 32 * tg;
+    const int nq = max(0, min(32, a.tb + a.ntok - tok0));  // of this wave's 32 tokens
+    // shares are cut at whole multiples of ut: workgroups with the same share
+    // index sweep the same keys at the same time, out of L2 (128 workgroups read
+    // a head's 4 MB of K and V at 4096 tokens)
+    const int t0 = (int)(u * ut), t1 = (int)min((u + 1) * ut, sq.tiles(jb));
+    // keys 0 .. last valid query position of the wave's tokens
+    const int L = P0 >= 0 && nq > 0 ? min(P0 + tok0 + nq - 1, pend - 1) + 1 : 0;
+    const int tlast = min(t1, (L + PF_KT - 1) / PF_KT);
+    const int qpos = P0 + tok0 + li;
+    const int qlim = li < nq && P0 >= 0 && qpos < pend ? qpos : -1;  // last key this lane's query attends to
+    // tiles that need no mask: below every query of 32 valid ones
+    const int tfull = nq == 32 && P0 >= 0 && P0 + tok0 + 31 < pend ? (P0 + tok0 + 1) / PF_KT : 0;
+
+    const uint32_t kvbytes = (uint32_t)a.pf_keys * (HD * 2), scbytes = (uint32_t)(a.pf_keys / PF_KT) * (PF_SC * 4);
+    const int64_t pair = (int64_t)bl * a.nkv + g;
+    const __amdgpu_buffer_rsrc_t rk = make_rsrc(a.kx + pair * kvbytes, kvbytes);
+    const __amdgpu_buffer_rsrc_t rv = make_rsrc(a.vx + pair * kvbytes, kvbytes);
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(reinterpret_cast<uint8_t*>(a.sx) + pair * scbytes, scbytes);
+    const uint32_t lane16 = lane * 16;
+    const int waves = 2 * G, per = (2 * KS + waves - 1) / waves;
+    // tile t -> its stage: 1 KB units dealt to the waves (`per` each, the last one
+    // repeated where they do not divide), the scales by every wave, so that all
+    // waves have the same number of loads in flight
+    auto issue = [&](int t) {
+        uint8_t* st = lds + (t & (NS - 1)) * ST;
+        for (int i = 0; i < per; ++i) {
+            const int x = min(wave + i * waves, 2 * KS - 1);
+            lds_dma16s(x < KS ? rk : rv, st + x * 1024, lane16, (uint32_t)t * KB + (x & (KS - 1)) * 1024);
+        }
+        if (lane < 32) lds_dma16s(rs, st + 2 * KB, lane16, (uint32_t)t * (PF_SC * 4));
+    };
+    if (t0 < t1) issue(t0);
+    if (t0 + 1 < t1) issue(t0 + 1);
+    f16x8 q[KS];
+    {
+        const int64_t row = (int64_t)b * a.T + min(tok0 + min(li, max(nq - 1, 0)), a.tb + a.ntok - 1) - a.row0;
+        const _Float16* qp = reinterpret_cast<const _Float16*>(a.qn) + (row * a.nh + h) * HD + 8 * hi;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) q[ks] = *reinterpret_cast<const f16x8*>(qp + 16 * ks);
+        // waited for here, so that no later wait of the compiler's counts the tile loads
+        __builtin_amdgcn_s_waitcnt(vm_wait(0));
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(q[ks]));
+    }
+    f32x16 acc[DT], s;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[dt][r] = 0.0f;
+    float m = -INFINITY, l = 0.0f;  // l: this lane's keys only
+
+    // S^T of a tile: element r of a lane is key 8 (r / 4) + 4 hi + r % 4 of
+    // query li.  Operands are read LA MFMAs ahead through a ring of
+    // registers, in this order: the LDS latency hides behind the matrix cores.
+    auto scores = [&](const uint8_t* kt) {
+        f16x8 f[LA + 1];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = 0.0f;
+#pragma unroll
+        for (int u = 0; u < LA; ++u) f[u] = *reinterpret_cast<const f16x8*>(kt + u * 1024);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < KS; ++u) {
+            if (u + LA < KS) f[(u + LA) % (LA + 1)] = *reinterpret_cast<const f16x8*>(kt + (u + LA) * 1024);
+            __builtin_amdgcn_sched_barrier(0);
+            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[u % (LA + 1)], q[u], s, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    // softmax and V product of tile t, whose scores are in s
+    auto update = [&](const uint8_t* vt, const float* sc, int t) {
+        const float thr = sc[64], m0 = m == -INFINITY ? 0.0f : m;
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+            const f32x4 k4 = *reinterpret_cast<const f32x4*>(sc + 8 * r4 + 4 * hi);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s[4 * r4 + r] = __builtin_fmaf(s[4 * r4 + r], k4[r], -m0);
+        }
+        // the first V units on their way under the softmax
+        f16x8 f[LA + 1];
+#pragma unroll
+        for (int u = 0; u < LA; ++u) f[u] = *reinterpret_cast<const f16x8*>(vt + u * 1024);
+        __builtin_amdgcn_sched_barrier(0);
+        if (t >= tfull) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                s[r] = PF_KT * t + 8 * (r >> 2) + 4 * hi + (r & 3) <= qlim ? s[r] : -INFINITY;
+        }
+        float mt = s[0];
+#pragma unroll
+        for (int r = 1; r < 16; ++r) mt = fmaxf(mt, s[r]);
+        mt = fmaxf(mt, __shfl_xor(mt, 32));
+        if (__any(mt > thr || m == -INFINITY)) {  // raise the running maximum (s is relative to m0)
+            const float up = m == -INFINITY ? ceilf(mt) : fmaxf(ceilf(mt), 0.0f);
+            const float corr = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(-up);
+            m = m0 + up;
+            l *= corr;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) acc[dt] = acc[dt] * corr;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = up == -INFINITY ? -INFINITY : s[r] - up;  // no key of this query yet
+        }
+        f16x8 pb[2];
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+            const f32x4 v4 = *reinterpret_cast<const f32x4*>(sc + 32 + 8 * r4 + 4 * hi);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float e = __builtin_amdgcn_exp2f(s[4 * r4 + r]);
+                l += e;
+                pb[r4 >> 1][4 * (r4 & 1) + r] = (_Float16)(e * v4[r]);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < KS; ++u) {
+            if (u + LA < KS) f[(u + LA) % (LA + 1)] = *reinterpret_cast<const f16x8*>(vt + (u + LA) * 1024);
+            __builtin_amdgcn_sched_barrier(0);
+            acc[u % DT] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[u % (LA + 1)], pb[u / DT], acc[u % DT], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    // Tile t is complete behind barrier t, and the stage that is filled behind
+    // it (t + 2's) is no longer read.  Group 0 passes barrier t before its scores
+    // of tile t, group 1 between its scores of tile t - 1 and the update with
+    // them; every wave passes t1 - t0 + 1 barriers.
+    auto pass = [&](int t) {
+        if (G == 4 && t + 1 < t1) __builtin_amdgcn_s_waitcnt(vm_wait(2 * KS / 8 + 1));  // all but tile t + 1's
+        else __builtin_amdgcn_s_waitcnt(vm_wait(0));
+        __syncthreads();
+        if (t + 2 < t1) issue(t + 2);
+    };
+    if (tg) pass(t0);
+    for (int t = t0; t < t1; ++t) {
+        if (!tg) pass(t);
+        const uint8_t* st = lds + (t & (NS - 1)) * ST;
+        if (t < tlast) scores(st + lane16);
+        if (tg) pass(t + 1);
+        if (t < tlast) update(st + KB + lane16, reinterpret_cast<const float*>(st + 2 * KB), t);
+    }
+    if (!tg) pass(t1);
+    l += __shfl_xor(l, 32);
+    __syncthreads();  // the stages are no longer read
+
+    // ---- rows: 16 at a time through the wave's own 16 KB, 16-byte chunks
+    // XOR-swizzled by row.  Rolled loops: this code runs once per workgroup, and
+    // unrolled (3400 instructions) its instruction fetches alone took 28 us ----
+    const bool lone = !pf_cut(a, n);
+    const float inv = lone ? (l > 0.0f ? 1.0f / l : 0.0f) : 1.0f;
+    float* piece = a.part + ((int64_t)slot * a.nkv + g) * pf_piece(G, HD);
+    if (!lone && hi == 0) {
+        float* ml = piece + G * PF_Q * HD + (w * PF_Q + 32 * tg + li) * 2;
+        ml[0] = m;
+        ml[1] = l;
+    }
+    piece += (w * PF_Q + 32 * tg) * HD;
+    constexpr int RL = HD / 4, RI = 64 / RL;  // lanes per row, rows per access
+    float* stg = reinterpret_cast<float*>(lds + wave * (16 * HD * 4));
+    const int esz = a.in_dt == DT_F32 ? 4 : 2, osz = a.out_dt == DT_F32 ? 4 : 2;
+    const bool gvec = ((uintptr_t)a.gate % (4 * esz)) == 0 && a.ld_in % 4 == 0 && a.q_hs % 4 == 0;
+    const bool ovec = ((uintptr_t)a.out % (4 * osz)) == 0 && a.ld_out % 4 == 0;
+#pragma unroll 1
+    for (int p = 0; p < 2; ++p) {
+        if ((li >> 4) == p) {
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int r4 = 0; r4 < 4; ++r4) {
+                    f32x4 y;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) y[r] = acc[dt][4 * r4 + r] * inv;
+                    *reinterpret_cast<f32x4*>(&stg[(li & 15) * HD + 4 * ((8 * dt + 2 * r4 + hi) ^ (li & 15))]) = y;
+                }
+        }
+        __builtin_amdgcn_wave_barrier();
+        constexpr int U = 4;  // accesses in flight
+#pragma unroll 1
+        for (int j0 = 0; j0 < 16; j0 += U * RI) {
+            const int d = 4 * (lane % RL);
+            f32x4 gt[U], y[U];
+#pragma unroll
+            for (int e = 0; e < U; ++e) {
+                const int rr = j0 + e * RI + lane / RL;  // row of the 16
+                y[e] = *reinterpret_cast<const f32x4*>(&stg[rr * HD + 4 * ((lane % RL) ^ rr)]);
+                gt[e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                if (!lone || 16 * p + rr >= nq) continue;
+                const int64_t gi = ((int64_t)b * a.T + tok0 + 16 * p + rr) * a.ld_in + (int64_t)h * a.q_hs + d;
+                if (gvec) {
+                    gt[e] = load_act4(a.gate, a.in_dt, gi);
+                } else {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) gt[e][c] = at_load(a.gate, a.in_dt, gi + c);
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < U; ++e) {
+                const int qr = 16 * p + j0 + e * RI + lane / RL;
+                if (!lone) {
+                    *reinterpret_cast<f32x4*>(piece + qr * HD + d) = y[e];
+                    continue;
+                }
+                if (qr >= nq) continue;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) y[e][c] *= 1.0f / (1.0f + __expf(-gt[e][c]));
+                const int64_t oi = ((int64_t)b * a.T + tok0 + qr) * a.ld_out + (int64_t)h * HD + d;
+                if (ovec) {
+                    store_act4(a.out, a.out_dt, oi, y[e]);
+                } else {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) store_act(a.out, a.out_dt, oi + c, y[e][c]);
+                }
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// Merges the shares of the blocks that were cut: one workgroup per (block, 16
+// of its tokens of a head, sequence), four rows per wave in flight together.
+template <int HD>
+__global__ __launch_bounds__(256) void attn_pf_merge(AttnArgs a) {
+    constexpr int E = HD / 64;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int h = blockIdx.y / (PF_Q / 16), bl = blockIdx.z, G = a.nh / a.nkv, g = h / G, w = h % G;
+    const uint32_t jb = blockIdx.x, ut = pf_longest(a);
+    const PfSeq sq(a, __builtin_amdgcn_readfirstlane(a.pos[a.b0 + bl]));
+    const int n = (int)pf_shares(sq, ut, jb);
+    if (!pf_cut(a, n)) return;
+    uint32_t slot = 0, units, cut;
+    for (int i = threadIdx.x & 63; i < bl && (uint32_t)bl > sq.nblk; i += 64) {  // lanes take sequences
+        const PfSeq o(a, a.pos[a.b0 + i]);
+        pf_count<false>(a, o, ut, o.nblk, units, cut);
+        slot += cut;
+    }
+    slot = pf_sum(slot);
+    for (int i = 0; i < bl && (uint32_t)bl <= sq.nblk; ++i) {  // lanes take blocks
+        const PfSeq o(a, __builtin_amdgcn_readfirstlane(a.pos[a.b0 + i]));
+        pf_count<true>(a, o, ut, o.nblk, units, cut);
+        slot += cut;
+    }
+    pf_count<true>(a, sq, ut, jb, units, cut);
+    slot += cut;
+    const int qb = (int)(sq.nblk - 1 - jb), nq = min(PF_Q, a.ntok - qb * PF_Q);
+    const int64_t ps = pf_piece(G, HD), next = ps * a.nkv;
+    const float* p0 = a.part + ((int64_t)slot * a.nkv + g) * ps;
+    const int qr = blockIdx.y % (PF_Q / 16) * 16 + wave * 4;
+    const float* ml = p0 + G * PF_Q * HD + (w * PF_Q + qr) * 2;
+    const float* src = p0 + (int64_t)(w * PF_Q + qr) * HD + lane * E;
+    float M[4], l[4], o[4][E];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        M[r] = -INFINITY;
+        l[r] = 0.0f;
+#pragma unroll
+        for (int e = 0; e < E; ++e) o[r][e] = 0.0f;
+    }
+    for (int i = 0; i < n; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) M[r] = fmaxf(M[r], ml[i * next + 2 * r]);
+    for (int i = 0; i < n; ++i) {
+        float x[4][E];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int e = 0; e < E; ++e) x[r][e] = src[i * next + r * HD + e];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float mi = ml[i * next + 2 * r];
+            const float wi = mi == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mi - M[r]);  // no key of this query in the share
+            l[r] += wi * ml[i * next + 2 * r + 1];
+#pragma unroll
+            for (int e = 0; e < E; ++e) o[r][e] += wi * x[r][e];
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        if (qr + r < nq)
+            gate_store<HD>(a, (a.b0 + bl) * a.T + a.tb + qb * PF_Q + qr + r, h, lane, o[r], l[r] > 0.0f ? 1.0f / l[r] : 0.0f);
+}
+
+// ---------------------------------------------------------------------------
 // decode over an INT8 cache on f16 MFMA: (key split, KV head g, row).  The
 // group's query heads are the MFMA columns (B = Q^T, 16 columns of which G
 // are used); a 64-key tile is staged as f16 once (K rows, V transposed) and
@@ -967,7 +1676,7 @@ __global__ __launch_bounds__(256) void attn_decode_i8h(AttnArgs a) {
             if (it <= G) {  // q or k: RMSNorm (1 + w), then RoPE on d < rot
                 float ss = 0.0f;
 #pragma unroll
-                for (int e = 0; e < E; ++e) ss += x[e] * x[e];
+                for (int e = 0; e < E; ++e) ss = __builtin_fmaf(x[e], x[e], ss);
                 ss = wave_sum(ss);
                 const float rms = sqrtf(ss / (float)HD + 1e-6f);
                 const float* w = isq ? a.qn_w : a.kn_w;
@@ -979,8 +1688,8 @@ __global__ __launch_bounds__(256) void attn_decode_i8h(AttnArgs a) {
                     if (d < a.rot) {
                         const float c = rc[d / 2], sn = rs[d / 2];
                         const float x0 = x[e], x1 = x[e + 1];
-                        x[e] = x0 * c - x1 * sn;
-                        x[e + 1] = x0 * sn + x1 * c;
+                        x[e] = rope0(x0, x1, c, sn);
+                        x[e + 1] = rope1(x0, x1, c, sn);
                     }
                 }
             }
@@ -1214,6 +1923,9 @@ size_t attn_bytes_per_row(int nh, int hd, int nsplit) {
     return (size_t)nh * hd * 4 + (size_t)nh * nsplit * (hd + 2) * 4;
 }
 
+size_t attn_pf_bytes_per_piece(int G, int hd) { return (size_t)G * PF_Q * (hd + 2) * 4; }
+size_t attn_pf_bytes_per_key(int hd) { return (size_t)2 * hd * 2 + PF_SC * 4 / PF_KT; }
+
 template <int HD>
 static void launch_combine(const AttnArgs& a, hipStream_t stream) {
     if (a.nsplit <= 1) return;
@@ -1224,7 +1936,13 @@ static void launch_combine(const AttnArgs& a, hipStream_t stream) {
 template <int HD>
 static hipError_t launch_attn_hd(const AttnArgs& a, hipStream_t stream) {
     if (a.prefill) {
-        hipLaunchKernelGGL(attn_prep<HD>, dim3(a.rows), dim3(64 * std::min(16, a.nh + 2 * a.nkv)), 0, stream, a);
+        launch_prep<HD>(a, stream);
+        if (a.pf_units) {
+            hipLaunchKernelGGL(attn_expand<HD>, dim3(a.pf_keys / PF_KT, a.nkv, a.nb), dim3(256), 0, stream, a);
+            hipLaunchKernelGGL(attn_pf<HD>, dim3(a.pf_grid), dim3(128 * (a.nh / a.nkv)), 0, stream, a);
+            hipLaunchKernelGGL(attn_pf_merge<HD>, dim3((a.ntok + PF_Q - 1) / PF_Q, a.nh * (PF_Q / 16), a.nb), dim3(256), 0, stream, a);
+            return hipGetLastError();
+        }
         // INT8: query blocks x key splits (f16 MFMA), merged by attn_combine;
         // FP32: one workgroup per query block over all its keys (FP32 MFMA)
         if (a.kv_dt == DT_I8) {
@@ -1241,7 +1959,7 @@ static hipError_t launch_attn_hd(const AttnArgs& a, hipStream_t stream) {
         else hipLaunchKernelGGL((attn_decode_i8h<HD, true, false>), dim3(a.nsplit, a.nkv, a.rows), dim3(256), 0, stream, a);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(attn_prep<HD>, dim3(a.rows), dim3(64 * std::min(16, a.nh + 2 * a.nkv)), 0, stream, a);
+    launch_prep<HD>(a, stream);
     if (a.kv_dt == DT_I8 && a.vcoal) hipLaunchKernelGGL((attn_decode_i8h<HD, false, true>), dim3(a.nsplit, a.nkv, a.rows), dim3(256), 0, stream, a);
     else if (a.kv_dt == DT_I8) hipLaunchKernelGGL((attn_decode_i8h<HD, false, false>), dim3(a.nsplit, a.nkv, a.rows), dim3(256), 0, stream, a);
     else hipLaunchKernelGGL((attn_split<HD, false>), dim3(a.nsplit, a.nkv, a.rows), dim3(256), 0, stream, a);

@@ -57,6 +57,16 @@ __device__ __forceinline__ void lds_dma16(__amdgpu_buffer_rsrc_t rs, uint8_t* ld
                  : "memory", "m0");
 }
 
+// The same with a scalar offset added (not range-checked: the caller keeps
+// soff + voff inside the buffer)
+__device__ __forceinline__ void lds_dma16s(__amdgpu_buffer_rsrc_t rs, uint8_t* lds_unit, uint32_t voff, uint32_t soff) {
+    const uint32_t m0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds_unit;
+    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :
+                 : "s"(m0), "v"(voff), "s"(rs), "s"(soff)
+                 : "memory", "m0");
+}
+
 // Epoch wrap of the persistent kernels' tagged hand-off words.  A word is
 // (tag << 32 | payload) with the launch epoch in the tag's high bits; once
 // the epoch's field wraps, a word written 2^bits launches earlier (a token

@@ -270,3 +270,55 @@ def test_attn_one_launch_decode_matches_three_launches(qw, oracle, io):
         assert torch.equal(o1[s], o0[s]), s
     for x1, x0 in zip(c1, c0):
         assert torch.equal(x1, x0)
+
+
+@pytest.mark.parametrize("hd,nh,nkv,B,T,starts,io,vmul", [
+    (256, 8, 2, 1, 32, [0], "f32", 1.0),          # the shortest run that takes it
+    (256, 8, 2, 1, 65, [700], "f32", 1.0),        # a one-token block behind a prefix, masked tiles in several shares
+    (256, 8, 2, 2, 300, [5, 600], "bf16", 1.0),   # ragged starts, blocks of several shares
+    (256, 8, 2, 5, 40, [0, 1, 31, 32, 33], "f16", 1.0),  # more sequences than blocks
+    (256, 8, 2, 70, 100, None, "f32", 1.0),       # more blocks than CUs: uncut blocks write the output themselves
+    (256, 6, 2, 1, 130, [17], "f32", 1.0),        # three query heads per KV head
+    (256, 2, 2, 2, 64, [0, 63], "f32", 1.0),      # one
+    (128, 8, 2, 2, 200, [0, 90], "f32", 1.0),
+    (256, 8, 2, 1, 150, [40], "f32", 1.0e6),      # V scales past the raise threshold's range
+    (256, 8, 2, 3, 64, [0, 900, 1000], "f32", 1.0),  # one sequence runs past the capacity
+])
+def test_attn_prefill_blocks(qw, oracle, relerr, hd, nh, nkv, B, T, starts, io, vmul):
+    """The 64-token-block INT8 prefill (expanded cache, shares, merge) against
+    the 16-token kernels (a context that keeps every run on them; those are
+    checked against the oracle above), over a cache with random codes behind the
+    starts: edges of blocks and tiles, head groups, unaligned rows (odd column
+    offset), the device error flag.  Both round q and p to f16 (2^-11) and sum
+    in FP32, p against different maxima: 1e-3 normwise of each other; the cache
+    written is the same kernel's and equal bit for bit."""
+    cap = 1024 if T < 1000 else T
+    starts = starts or [(37 * b) % 500 for b in range(B)]
+    st = Stream(oracle, B, T, 900 + T + hd, hd=hd, nh=nh, nkv=nkv)
+    tdt = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}[io]
+    rows = dev(st.rows.reshape(B * T, -1))
+    rows[:, nh * 2 * hd + nkv * hd:] *= vmul
+    for pad in (0, 1):
+        wide = torch.zeros(B * T, st.ld + 4, device="cuda", dtype=tdt)
+        wide[:, pad:pad + st.ld] = rows.to(tdt)
+        gen = torch.Generator(device="cuda").manual_seed(3)
+        first = qw.kv_cache(B, cap, nkv, hd)
+        for c in first[:2]:
+            c.copy_(torch.randint(-127, 128, c.shape, generator=gen, device="cuda", dtype=torch.int8))
+        for c, m in zip(first[2:], (1.0, vmul)):
+            c.copy_(torch.rand(c.shape, generator=gen, device="cuda") * 0.02 * m + 0.001)
+        outs, caches, flags = [], [], []
+        for env in ({}, {"QW_ATTN_PF_MIN": "1000000"}):
+            c = _ctx_with(qw, env)
+            cache = tuple(x.clone() for x in first)
+            outs.append(run_gpu(qw, c, st, cache, wide[:, pad:], starts, T, 1.0e7, hd // 4,
+                                out_dtype=torch.float32 if vmul > 1 else tdt, max_len=cap))
+            flags.append(c.device_error())
+            torch.cuda.synchronize()
+            caches.append(cache)
+            c.close()
+        assert flags[0] == flags[1] and (flags[0] != 0) == any(s + T > cap for s in starts)
+        assert all(torch.equal(x, y) for x, y in zip(*caches))
+        err = relerr(host(outs[0]), host(outs[1]))
+        print("blocks", hd, nh, nkv, B, T, pad, err)
+        assert err <= (1e-3 if io == "f32" else 8e-3 if io == "bf16" else 2e-3), err
