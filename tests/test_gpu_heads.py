@@ -192,6 +192,24 @@ def test_rmsnorm(qw, ctx, oracle, relerr, M, K):
     assert relerr(host(y), oracle.rmsnorm_f64(x, w)) <= 1e-6
 
 
+@pytest.mark.parametrize("M,K,pad", [(5, 4, 0), (1023, 1024, 0), (1025, 1028, 0), (3, 4096, 0), (6, 1024, 1), (2, 102, 0)])
+@pytest.mark.parametrize("xdt,ydt", [("float32", "bfloat16"), ("float32", "float16"), ("bfloat16", "float32")])
+def test_rmsnorm_rows(qw, ctx, M, K, pad, xdt, ydt):
+    """The wave-per-row kernel (both workgroup sizes, both register widths, a
+    ragged last chunk) and the rows it leaves to the general one (misaligned
+    base, K not a multiple of 4) against float64; bar: one rounding of the
+    output type plus 1e-6 for the FP32 sum."""
+    gen = torch.Generator().manual_seed(M * 7 + K)
+    x = (torch.randn(M * K + pad, generator=gen) * 2.0).to(getattr(torch, xdt)).cuda()[pad:].view(M, K)
+    w = (torch.randn(K, generator=gen) * 0.1).cuda()
+    y = torch.empty(M, K, device="cuda", dtype=getattr(torch, ydt))
+    qw.rmsnorm(ctx, x, w, y)
+    torch.cuda.synchronize()
+    ref = x.double() / torch.sqrt(x.double().square().mean(1, keepdim=True) + 1e-6) * (1.0 + w.double())
+    ulp = {"float32": 0.0, "float16": 2.0 ** -11, "bfloat16": 2.0 ** -8}[ydt]
+    assert ((y.double() - ref).abs() <= (ulp + 1e-6) * ref.abs() + 1e-7).all()
+
+
 def test_rmsnorm_constant_closed_form(qw, ctx, oracle):
     """x = c everywhere: y = c / sqrt(c^2 + eps) * (1 + w)."""
     K, c = 1024, 0.75
