@@ -167,6 +167,14 @@ __device__ __forceinline__ float wave_sum_to_lane63(float v) {
     return v;
 }
 
+// Workgroup ids go round robin to the 8 XCDs; position of workgroup b in an
+// order that gives every XCD one contiguous run (the first n % 8 XCDs one more
+// than the others), so that blocks that share operands meet in one L2.
+__device__ __forceinline__ int xcd_run(int b, int n) {
+    const int x = b & 7, rem = n & 7;
+    return x * (n >> 3) + min(x, rem) + (b >> 3);
+}
+
 __device__ __forceinline__ float silu_f(float v) { return v / (1.0f + __expf(-v)); }
 
 // Orderable key of (value, index): larger value wins, then LOWER index wins.

@@ -131,7 +131,7 @@ void gemm_kernel(GemmArgs a) {
     // share a weight block run on the same L2.
     const int nwg = gridDim.x;
     int b = blockIdx.x;
-    if ((nwg & 7) == 0) b = (b & 7) * (nwg >> 3) + (b >> 3);
+    b = xcd_run(b, nwg);
     // split-K (64-row blocks only): consecutive ids after the XCD order are
     // the splits of one tile
     constexpr bool SPLITK = RW == 64 && !ARGMAX;

@@ -176,7 +176,7 @@ __global__ __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) void gemm_da_kernel(Gem
     // the grouped raster
     const int nwg = gridDim.x;
     int b = blockIdx.x;
-    if ((nwg & 7) == 0) b = (b & 7) * (nwg >> 3) + (b >> 3);
+    b = xcd_run(b, nwg);
     const int S = PART ? a.splitk : 1;
     const int sk = PART ? b % S : 0;
     if constexpr (PART) b /= S;
