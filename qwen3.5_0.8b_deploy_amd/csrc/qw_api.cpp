@@ -1327,14 +1327,19 @@ qw_status qw_attn_forward(qw_ctx* ctx, const qw_attn_params* p, const qw_kv_cach
             a.split = std::max(256, (s8 + 31) / 32 * 32);
             a.nsplit = (len + a.split - 1) / a.split;
         } else {
+            // about 2.5 workgroups per CU, at most 8 shares of >= 128 keys
+            const int64_t wgs = (int64_t)batch * nkv * ((tokens + 15) / 16);
             a.split = len;
-            a.nsplit = 1;
+            a.nsplit = (int)std::max<int64_t>(1, std::min<int64_t>({(int64_t)5 * ctx->num_cus / 2 / wgs, (int64_t)8,
+                                                                    (int64_t)(len + 127) / 128}));
+            a.blk = 16;
         }
+        a.lim = cache->dtype == QW_I8 ? a.nsplit * a.split : len;
         // INT8, longer runs: 32-token query blocks over the cache expanded to
         // f16 MFMA operands once per segment (attn_pf), wherever the workspace
         // holds the expanded keys and a segment of rows
         if (cache->dtype == QW_I8 && tokens >= ctx->attn_pf_min) {
-            const int64_t keys = (std::min<int64_t>(cache->capacity, (int64_t)a.nsplit * a.split) + 63) / 64 * 64;
+            const int64_t keys = (std::min<int64_t>(cache->capacity, a.lim) + 63) / 64 * 64;
             const size_t kvb = (size_t)nkv * keys * qwk::attn_pf_bytes_per_key(hd);
             const size_t row = (size_t)nh * hd * 2, piece = qwk::attn_pf_bytes_per_piece(nh / nkv, hd);
             int min_units = std::min(ctx->num_cus, 32);
@@ -1437,6 +1442,7 @@ qw_status qw_attn_forward(qw_ctx* ctx, const qw_attn_params* p, const qw_kv_cach
     if (seg < 1) return fail(ctx, QW_ERR_WORKSPACE, "attn: workspace too small for one row");
     a.split = split;
     a.nsplit = nsplit;
+    a.lim = nsplit * split;
     // one new token per sequence over an INT8 cache: one launch per segment
     // (q/k/v preparation and the split merge inside the attention kernel)
     // when the launch is small (at most 16 splits: one wave merges a head's

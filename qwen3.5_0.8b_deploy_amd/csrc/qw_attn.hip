@@ -104,7 +104,7 @@ __global__ __launch_bounds__(1024) void attn_prep(AttnArgs a) {
     const int b = r / a.T, t = r % a.T;
     const int P = a.pos[b] + t;
     // a position outside the cache, or past the keys the launch was sized for
-    const bool ok = P >= 0 && P < a.cap && P < a.nsplit * a.split;
+    const bool ok = P >= 0 && P < a.cap && P < a.lim;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     if (!ok && threadIdx.x == 0) *a.err = 1u;
     // the rotation of this position, shared by every q and k head
@@ -192,7 +192,7 @@ __global__ __launch_bounds__(1024) void attn_prep_rows(AttnArgs a) {
         return a.pos[b] + r % a.T;
     };
     // a position outside the cache, or past the keys the launch was sized for
-    auto valid = [&](int P) { return P >= 0 && P < a.cap && P < a.nsplit * a.split; };
+    auto valid = [&](int P) { return P >= 0 && P < a.cap && P < a.lim; };
     for (int it0 = 0; it0 < items; it0 += blockDim.x >> 6) {
         const int it = it0 + wave;
         const bool isq = it < a.nh, isk = !isq && it < a.nh + a.nkv;
@@ -313,7 +313,7 @@ __global__ __launch_bounds__(256) void attn_split(AttnArgs a) {
     const int s = blockIdx.x, g = blockIdx.y, rl = blockIdx.z, r = a.row0 + rl;
     const int b = r / a.T, t = r % a.T;
     const int P = a.pos[b] + t;
-    const int L = (P >= 0 && P < a.cap && P < a.nsplit * a.split) ? P + 1 : 0;  // causal: keys 0 .. P
+    const int L = (P >= 0 && P < a.cap && P < a.lim) ? P + 1 : 0;  // causal: keys 0 .. P
     const int k0 = s * a.split, k1 = min(k0 + a.split, L);
     const int G = a.nh / a.nkv;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -520,6 +520,11 @@ __device__ __forceinline__ void gate_store(const AttnArgs& a, int r, int h, int 
 // DC > 1 (many splits): blockIdx.z takes HD/DC of the head's dims, so more
 // workgroups share the split partials' reads (each recomputes M and l from
 // the splits' two floats).
+// Keys per share of a query block with L keys (the FP32 query-block kernel).
+__device__ __forceinline__ int block_share(const AttnArgs& a, int L) {
+    return max(128, ((L + a.nsplit - 1) / a.nsplit + AT_KT - 1) / AT_KT * AT_KT);
+}
+
 template <int HD, int NW, int DC = 1>
 __global__ __launch_bounds__(64 * NW) void attn_combine(AttnArgs a) {
     static_assert(DC == 1 || NW > 1, "dim chunks with the multi-wave merge");
@@ -528,9 +533,16 @@ __global__ __launch_bounds__(64 * NW) void attn_combine(AttnArgs a) {
     const int rl = blockIdx.x, h = blockIdx.y, r = a.row0 + rl;
     const int b = r / a.T, t = r % a.T;
     const int P = a.pos[b] + t;
-    const int L = (P >= 0 && P < a.cap && P < a.nsplit * a.split) ? P + 1 : 0;
+    const int L = (P >= 0 && P < a.cap && P < a.lim) ? P + 1 : 0;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int ns = (L + a.split - 1) / a.split;
+    int split = a.split;
+    if (a.blk) {  // cut by blocks: the keys of this row's block
+        const int last = min(a.tb + (t - a.tb) / a.blk * a.blk + a.blk, a.tb + a.ntok) - 1;
+        const int Lb = P - t >= 0 ? min(P - t + last, min(a.cap, a.lim) - 1) + 1 : 0;
+        split = block_share(a, Lb);
+        if (Lb <= split) return;  // one share: the row is written
+    }
+    const int ns = (L + split - 1) / split;
     const float* pp = a.part + ((int64_t)rl * a.nh + h) * a.nsplit * (HD + 2);
     __shared__ float red[2][NW];
     __shared__ __attribute__((aligned(16))) float osum[NW][HD / DC];
@@ -612,13 +624,20 @@ __global__ __launch_bounds__(64 * NW) void attn_combine(AttnArgs a) {
 //   S^T = K Q^T (32 keys x 16 queries per tile; Q in registers as the B
 //   operand), causal mask, online softmax per query column, O^T += V^T P^T
 //   (P^T is the score tile's own D layout: the B operand needs no shuffle).
-// K and V tiles of 32 keys are staged in LDS once for the KV group (INT8
-// codes with their scales folded into the scores and probabilities, or FP32).
-template <int HD, bool I8>
-__global__ __launch_bounds__(256) void attn_prefill(AttnArgs a) {
-    using Tl = AtTile<HD, I8>;
-    constexpr int ESZ = I8 ? 1 : 4, CPR = HD * ESZ / 16, KB = HD / 16, DT = HD / 16;
-    const int qb = blockIdx.x, g = blockIdx.y, b = a.b0 + blockIdx.z;
+// K and V tiles of 32 keys of the FP32 cache are staged in LDS once for the KV
+// group, each under the other's product.
+// Bound: the FP32 matrix cores (256 MFMAs of 32 cycles per wave and tile).  A
+// block's keys are cut into up to a.nsplit equal shares (at least 128 keys; the
+// number is chosen for about 2.5 workgroups per CU), merged by attn_combine:
+// without, 2 x 600 tokens make 152 workgroups, one per CU and the longest alone
+// at the end (317 -> 135 us, and 15 for the merge; without the cut 25.6 -> 15.7 us
+// at 8 x 21 tokens, from the V rows spread over the LDS banks and 16-byte gates).
+template <int HD>
+__global__ __launch_bounds__(256, 2) void attn_prefill(AttnArgs a) {
+    constexpr int ROW = HD + 4;                // LDS row stride, floats (bank spread)
+    constexpr int PER = AT_KT * HD / 4 / 256;  // 16-byte chunks of a K (or V) tile per thread
+    constexpr int KB = HD / 16, DT = HD / 16;
+    const int qb = blockIdx.x / a.nsplit, sp = blockIdx.x % a.nsplit, g = blockIdx.y, b = a.b0 + blockIdx.z;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
     const int G = a.nh / a.nkv;
     const int h = g * G + min(wave, G - 1);
@@ -626,36 +645,38 @@ __global__ __launch_bounds__(256) void attn_prefill(AttnArgs a) {
     const int P0 = a.pos[b];
     const int nq = min(16, a.tb + a.ntok - tok0);          // valid queries of the block
     const int plast = P0 + tok0 + nq - 1;                  // last query position
-    const int pend = min(a.cap, a.nsplit * a.split);       // positions must stay below this
+    const int pend = min(a.cap, a.lim);       // positions must stay below this
     const int L = P0 >= 0 ? min(plast, pend - 1) + 1 : 0;  // keys 0 .. last valid query position
     const int qpos = P0 + tok0 + li;                       // this lane's query position
     const bool qvalid = li < nq && P0 >= 0 && qpos < pend; // an invalid query outputs zeros
+    // this workgroup's share of the keys: [k0, k1)
+    const int share = block_share(a, L), k0 = sp * share, k1 = min(k0 + share, L);
+    if (k0 >= k1 && sp > 0) return;  // uniform; the first share of a flagged block still writes zeros
+    const bool lone = L <= share;
 
-    __shared__ __attribute__((aligned(16))) uint8_t Kt[AT_KT * Tl::KROW];
-    __shared__ __attribute__((aligned(16))) uint8_t Vt[AT_KT * Tl::VROW];
-    __shared__ float ksc[AT_KT], vsc[AT_KT];
+    __shared__ __attribute__((aligned(16))) float Kt[AT_KT * ROW], Vt[AT_KT * ROW];
 
-    const uint8_t* kbase = reinterpret_cast<const uint8_t*>(a.kc);
-    const uint8_t* vbase = reinterpret_cast<const uint8_t*>(a.vc);
     const int64_t slot0 = (int64_t)b * a.cap * a.nkv + g;
-    u32x4 pre[Tl::PER];
-    float psc = 0.0f;
-    auto issue = [&](int kt) {
-        const int n = min(AT_KT, L - kt);
+    // one register set for both: K of the next tile is on its way under the
+    // V product, V under the scores
+    f32x4 pre[PER];
+    auto issue = [&](const void* base, int kt) {
+        const int n = min(AT_KT, k1 - kt);
 #pragma unroll
-        for (int i = 0; i < Tl::PER; ++i) {
-            const int c = threadIdx.x + 256 * i, isv = c >= Tl::CH, cc = c - isv * Tl::CH;
-            const int j = cc / CPR, part = cc % CPR;
-            const int64_t slot = slot0 + (int64_t)(kt + j) * a.nkv;
-            if (j < n) pre[i] = *reinterpret_cast<const u32x4*>((isv ? vbase : kbase) + slot * (HD * ESZ) + part * 16);
-            else pre[i] = u32x4{0u, 0u, 0u, 0u};
-        }
-        if (I8 && threadIdx.x < 2 * AT_KT) {
-            const int j = threadIdx.x & (AT_KT - 1);
-            psc = j < n ? (threadIdx.x < AT_KT ? a.ks : a.vs)[slot0 + (int64_t)(kt + j) * a.nkv] : 0.0f;
+        for (int i = 0; i < PER; ++i) {
+            const int c = threadIdx.x + 256 * i, j = c / (HD / 4), part = c % (HD / 4);
+            pre[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            if (j < n) pre[i] = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(base) + (slot0 + (int64_t)(kt + j) * a.nkv) * HD + part * 4);
         }
     };
-    if (L > 0) issue(0);
+    auto stage = [&](float* tile) {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int c = threadIdx.x + 256 * i, j = c / (HD / 4), part = c % (HD / 4);
+            *reinterpret_cast<f32x4*>(&tile[j * ROW + part * 4]) = pre[i];
+        }
+    };
+    if (k0 < k1) issue(a.kc, k0);
 
     // Q block of this wave's head in registers: lane (lg, li) holds Q[li][16kb + 4lg + q]
     f32x4 qr[KB];
@@ -671,107 +692,115 @@ __global__ __launch_bounds__(256) void attn_prefill(AttnArgs a) {
     for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     float m = -INFINITY, l = 0.0f;
 
-    for (int kt = 0; kt < L; kt += AT_KT) {
-        __syncthreads();  // the previous tile is consumed
-#pragma unroll
-        for (int i = 0; i < Tl::PER; ++i) {
-            const int c = threadIdx.x + 256 * i, isv = c >= Tl::CH, cc = c - isv * Tl::CH;
-            const int j = cc / CPR, part = cc % CPR;
-            if (isv) {
-                *reinterpret_cast<u32x4*>(&Vt[j * Tl::VROW + part * 16]) = pre[i];
-            } else {
-                uint32_t* d32 = reinterpret_cast<uint32_t*>(&Kt[j * Tl::KROW + part * 16]);
-                d32[0] = pre[i][0]; d32[1] = pre[i][1]; d32[2] = pre[i][2]; d32[3] = pre[i][3];
-            }
-        }
-        if (I8 && threadIdx.x < 2 * AT_KT) (threadIdx.x < AT_KT ? ksc : vsc)[threadIdx.x & (AT_KT - 1)] = psc;
-        if (kt + AT_KT < L) issue(kt + AT_KT);
+    for (int kt = k0; kt < k1; kt += AT_KT) {
+        stage(Kt);  // (the waves are past the previous scores)
+        issue(a.vc, kt);
         __syncthreads();
-        if (wave >= G) continue;
         // S^T for keys kt + 16*sub + (4lg + r), queries li
-        f32x4 sc[2];
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub) {
-            f32x4 sacc = {0.0f, 0.0f, 0.0f, 0.0f};
-            const int key = 16 * sub + li;  // A operand row: key, k = dim
-#pragma unroll
-            for (int kb = 0; kb < KB; ++kb) {
-                float k4[4];
-                if (I8) {
-                    const uint32_t c4 = *reinterpret_cast<const uint32_t*>(&Kt[key * Tl::KROW + 16 * kb + 4 * lg]);
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) k4[q] = (float)(int8_t)((c4 >> (8 * q)) & 0xff);
-                } else {
-                    const f32x4 kv = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(&Kt[key * Tl::KROW]) + 16 * kb + 4 * lg);
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) k4[q] = kv[q];
-                }
-#pragma unroll
-                for (int q = 0; q < 4; ++q) sacc = at_mfma16(k4[q], qr[kb][q], sacc);
-            }
-            sc[sub] = sacc;
-        }
-        // scale, mask, running max per query column li
-        float mt = -INFINITY;
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int kl = 16 * sub + 4 * lg + r, kp = kt + kl;
-                float v = sc[sub][r] * scale * (I8 ? ksc[kl] : 1.0f);
-                v = (qvalid && kp <= qpos && kp < L) ? v : -INFINITY;
-                sc[sub][r] = v;
-                mt = fmaxf(mt, v);
-            }
-        mt = fmaxf(mt, __shfl_xor(mt, 16));
-        mt = fmaxf(mt, __shfl_xor(mt, 32));
-        const float mn = fmaxf(m, mt);
-        const float corr = mn == -INFINITY ? 1.0f : __expf(m - mn);
-        float ps = 0.0f;
         f32x4 pb[2];
+        float corr = 1.0f;
+        if (wave < G) {
+            f32x4 sc[2];
 #pragma unroll
-        for (int sub = 0; sub < 2; ++sub)
+            for (int sub = 0; sub < 2; ++sub) {
+                f32x4 sacc = {0.0f, 0.0f, 0.0f, 0.0f};
+                const float* kr = &Kt[(16 * sub + li) * ROW + 4 * lg];  // A operand row: key, k = dim
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int kl = 16 * sub + 4 * lg + r;
-                const float p = mn == -INFINITY ? 0.0f : __expf(sc[sub][r] - mn);
-                ps += p;
-                pb[sub][r] = I8 ? p * vsc[kl] : p;  // B operand of P V: (key 4lg+r, query li)
-            }
-        ps += __shfl_xor(ps, 16);
-        ps += __shfl_xor(ps, 32);
-        l = l * corr + ps;
-        m = mn;
+                for (int kb = 0; kb < KB; ++kb) {
+                    const f32x4 k4 = *reinterpret_cast<const f32x4*>(kr + 16 * kb);
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) acc[dt] = acc[dt] * corr;
-        // O^T[d][query] += V^T[d][key] P^T[key][query]
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int key = 16 * sub + 4 * lg + q, d = 16 * dt + li;
-                    const float va = I8 ? (float)(int8_t)Vt[key * Tl::VROW + d]
-                                        : reinterpret_cast<const float*>(&Vt[key * Tl::VROW])[d];
-                    acc[dt] = at_mfma16(va, pb[sub][q], acc[dt]);
+                    for (int q = 0; q < 4; ++q) sacc = at_mfma16(k4[q], qr[kb][q], sacc);
                 }
+                sc[sub] = sacc;
+            }
+            // scale, mask, running max per query column li
+            float mt = -INFINITY;
+#pragma unroll
+            for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int kp = kt + 16 * sub + 4 * lg + r;
+                    const float v = qvalid && kp <= qpos && kp < k1 ? sc[sub][r] * scale : -INFINITY;
+                    sc[sub][r] = v;
+                    mt = fmaxf(mt, v);
+                }
+            mt = fmaxf(mt, __shfl_xor(mt, 16));
+            mt = fmaxf(mt, __shfl_xor(mt, 32));
+            const float mn = fmaxf(m, mt);
+            corr = mn == -INFINITY ? 1.0f : __expf(m - mn);
+            float ps = 0.0f;
+#pragma unroll
+            for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float p = mn == -INFINITY ? 0.0f : __expf(sc[sub][r] - mn);
+                    ps += p;
+                    pb[sub][r] = p;  // B operand of P V: (key 4lg+r, query li)
+                }
+            ps += __shfl_xor(ps, 16);
+            ps += __shfl_xor(ps, 32);
+            l = l * corr + ps;
+            m = mn;
+        }
+        stage(Vt);  // (the waves are past the previous V product)
+        if (kt + AT_KT < k1) issue(a.kc, kt + AT_KT);
+        __syncthreads();
+        if (wave < G) {
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) acc[dt] = acc[dt] * corr;
+            // O^T[d][query] += V^T[d][key] P^T[key][query]
+#pragma unroll
+            for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        acc[dt] = at_mfma16(Vt[(16 * sub + 4 * lg + q) * ROW + 16 * dt + li], pb[sub][q], acc[dt]);
+        }
     }
     if (wave >= G || li >= nq) return;
     // acc[dt] lane (lg, li) element r: O^T[16dt + 4lg + r][query li]
     const int64_t r = (int64_t)b * a.T + tok0 + li;
+    if (!lone) {  // a partial (o, max, sum) for the combine kernel
+        if (!qvalid || qpos < k0) return;  // never read for this query
+        float* dst = a.part + (((r - a.row0) * a.nh + h) * a.nsplit + sp) * (HD + 2);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) dst[16 * dt + 4 * lg + rr] = acc[dt][rr];
+        if (lg == 0) {
+            dst[HD] = m;
+            dst[HD + 1] = l;
+        }
+        return;
+    }
     const float inv = L > 0 && l > 0.0f ? 1.0f / l : 0.0f;
+    const int esz = a.in_dt == DT_F32 ? 4 : 2, osz = a.out_dt == DT_F32 ? 4 : 2;
+    const bool vec = ((uintptr_t)a.gate % (4 * esz)) == 0 && a.ld_in % 4 == 0 && a.q_hs % 4 == 0 &&
+                     ((uintptr_t)a.out % (4 * osz)) == 0 && a.ld_out % 4 == 0;
+    const int64_t gi = r * a.ld_in + (int64_t)h * a.q_hs + 4 * lg, oi = r * a.ld_out + (int64_t)h * HD + 4 * lg;
+    if (vec) {
+#pragma unroll
+        for (int d0 = 0; d0 < DT; d0 += 4) {
+            f32x4 gt[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) gt[e] = load_act4(a.gate, a.in_dt, gi + 16 * (d0 + e));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                f32x4 y;
+#pragma unroll
+                for (int rr = 0; rr < 4; ++rr) y[rr] = acc[d0 + e][rr] * inv * (1.0f / (1.0f + __expf(-gt[e][rr])));
+                store_act4(a.out, a.out_dt, oi + 16 * (d0 + e), y);
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-            const int d = 16 * dt + 4 * lg + rr;
-            const float gt = at_load(a.gate, a.in_dt, r * a.ld_in + (int64_t)h * a.q_hs + d);
-            const float y = acc[dt][rr] * inv * (1.0f / (1.0f + __expf(-gt)));
-            const int64_t oi = r * a.ld_out + (int64_t)h * HD + d;
-            if (a.out_dt == DT_F32) reinterpret_cast<float*>(a.out)[oi] = y;
-            else store_act(a.out, a.out_dt, oi, y);
-        }
+        for (int rr = 0; rr < 4; ++rr)
+            store_act(a.out, a.out_dt, oi + 16 * dt + rr,
+                      acc[dt][rr] * inv * (1.0f / (1.0f + __expf(-at_load(a.gate, a.in_dt, gi + 16 * dt + rr)))));
 }
 
 // ---------------------------------------------------------------------------
@@ -829,7 +858,7 @@ __global__ __launch_bounds__(256) void attn_prefill_i8h(AttnArgs a) {
     const int P0 = a.pos[b];
     const int nq = min(16, a.tb + a.ntok - tok0);
     const int plast = P0 + tok0 + nq - 1;
-    const int pend = min(a.cap, a.nsplit * a.split);
+    const int pend = min(a.cap, a.lim);
     const int L = P0 >= 0 ? min(plast, pend - 1) + 1 : 0;
     const int qpos = P0 + tok0 + li;
     const bool qvalid = li < nq && P0 >= 0 && qpos < pend;
@@ -1057,7 +1086,7 @@ __device__ __forceinline__ uint32_t pf_uni(uint32_t v) { return __builtin_amdgcn
 struct PfSeq {
     uint32_t nblk, c, tmax;
     __device__ __forceinline__ PfSeq(const AttnArgs& a, int P0) {
-        const int pend = min(a.cap, a.nsplit * a.split);
+        const int pend = min(a.cap, a.lim);
         nblk = (a.ntok + PF_Q - 1) / PF_Q;
         tmax = (uint32_t)(pend + PF_KT - 1) / PF_KT;
         c = (uint32_t)(min(max(P0, 0), pend) + a.tb + PF_KT - 1) / PF_KT;
@@ -1166,7 +1195,7 @@ __global__ __launch_bounds__(256) void attn_expand(AttnArgs a) {
     constexpr int KS = HD / 16, DT = HD / 32;
     const int tile = blockIdx.x, g = blockIdx.y, b = a.b0 + blockIdx.z;
     const int P0 = a.pos[b];
-    const int total = min(P0 + a.tb + a.ntok, min(a.cap, a.nsplit * a.split));  // keys in the cache after attn_prep
+    const int total = min(P0 + a.tb + a.ntok, min(a.cap, a.lim));  // keys in the cache after attn_prep
     const int k0 = tile * PF_KT;
     if (P0 < 0 || k0 >= total) return;
     const int nk = min(PF_KT, total - k0);
@@ -1258,7 +1287,7 @@ __global__ __launch_bounds__(512, 2) void attn_pf(AttnArgs a) {
     }
     if (n == 0) return;  // past the last unit; uniform
     const int qb = (int)(sq.nblk - 1 - jb);
-    const int pend = min(a.cap, a.nsplit * a.split);
+    const int pend = min(a.cap, a.lim);
     const int b = a.b0 + bl, h = g * G + w, tok0 = a.tb + qb * PF_Q + 32 * tg;
     const int nq = max(0, min(32, a.tb + a.ntok - tok0));  // of this wave's 32 tokens
     // shares are cut at whole multiples of ut: workgroups with the same share
@@ -1582,7 +1611,7 @@ __global__ __launch_bounds__(256) void attn_decode_i8h(AttnArgs a) {
     const int s = blockIdx.x, g = blockIdx.y, rl = blockIdx.z, r = a.row0 + rl;
     const int b = r / a.T, t = r % a.T;
     const int P = a.pos[b] + t;
-    const int L = (P >= 0 && P < a.cap && P < a.nsplit * a.split) ? P + 1 : 0;
+    const int L = (P >= 0 && P < a.cap && P < a.lim) ? P + 1 : 0;
     const int k0 = s * a.split, k1 = min(k0 + a.split, L);
     const int G = a.nh / a.nkv;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
@@ -1944,13 +1973,15 @@ static hipError_t launch_attn_hd(const AttnArgs& a, hipStream_t stream) {
             return hipGetLastError();
         }
         // INT8: query blocks x key splits (f16 MFMA), merged by attn_combine;
-        // FP32: one workgroup per query block over all its keys (FP32 MFMA)
+        // FP32: the same on FP32 MFMA, the keys cut by blocks
         if (a.kv_dt == DT_I8) {
             hipLaunchKernelGGL(attn_prefill_i8h<HD>, dim3((a.ntok + 15) / 16 * a.nsplit, a.nkv, a.nb), dim3(256), 0,
                                stream, a);
             launch_combine<HD>(a, stream);
         } else {
-            hipLaunchKernelGGL((attn_prefill<HD, false>), dim3((a.ntok + 15) / 16, a.nkv, a.nb), dim3(256), 0, stream, a);
+            hipLaunchKernelGGL((attn_prefill<HD>), dim3((a.ntok + 15) / 16 * a.nsplit, a.nkv, a.nb), dim3(256), 0,
+                               stream, a);
+            launch_combine<HD>(a, stream);
         }
         return hipGetLastError();
     }

@@ -337,6 +337,8 @@ struct AttnArgs {
     float* qn;             // workspace [rows][nh][hd]: normalized, rotated q
     float* part;           // workspace [rows][nh][nsplit][hd + 2]: split partials
     int split, nsplit;     // keys per split, splits per row (upper bound)
+    int lim;               // positions must stay below this (the keys the launch was sized for)
+    int blk;               // FP32 prefill: the keys are cut per block of this many tokens (0: by `split`)
     int prefill;           // query-block kernel: tokens [tb, tb + ntok) of sequences [b0, b0 + nb)
     int b0, nb, tb, ntok;  // (the rows of the segment are then contiguous: row0 = b0*T + tb)
     unsigned* cnt;         // one-launch decode (T == 1, INT8): arrival counters [rows][nkv], zero between launches

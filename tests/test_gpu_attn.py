@@ -322,3 +322,39 @@ def test_attn_prefill_blocks(qw, oracle, relerr, hd, nh, nkv, B, T, starts, io, 
         err = relerr(host(outs[0]), host(outs[1]))
         print("blocks", hd, nh, nkv, B, T, pad, err)
         assert err <= (1e-3 if io == "f32" else 8e-3 if io == "bf16" else 2e-3), err
+
+
+@pytest.mark.parametrize("B,T,cap,starts,hd,io", [
+    (1, 16, 600, [500], 256, "f32"),           # one block, its keys cut
+    (1, 300, 1024, [700], 256, "f32"),         # up to the last cache slot
+    (2, 90, 700, [0, 600], 256, "bf16"),       # one share and several in one launch, ragged blocks
+    (1, 200, 900, [650], 128, "f32"),
+    (2, 64, 640, [100, 600], 256, "f32"),      # the second sequence runs past the capacity
+])
+def test_attn_prefill_f32_shares(qw, oracle, relerr, B, T, cap, starts, hd, io):
+    """The FP32 query-block kernel with its keys cut into shares against the
+    key-split row kernel (a context that sends every run to it), over a random
+    cache; rows with an odd column offset take the element accesses.  FP32
+    throughout: 2e-5 normwise (BF16 outputs: one rounding)."""
+    st = Stream(oracle, B, T, 1700 + T, hd=hd)
+    tdt = {"f32": torch.float32, "bf16": torch.bfloat16}[io]
+    for pad in (0, 1):
+        wide = torch.zeros(B * T, st.ld + 4, device="cuda", dtype=tdt)
+        wide[:, pad:pad + st.ld] = dev(st.rows.reshape(B * T, -1)).to(tdt)
+        gen = torch.Generator(device="cuda").manual_seed(5)
+        first = [torch.randn(B, cap, 2, hd, generator=gen, device="cuda") for _ in range(2)]
+        outs, caches, flags = [], [], []
+        for env in ({}, {"QW_ATTN_PREFILL_MIN": "100000"}):
+            c = _ctx_with(qw, env)
+            zero = torch.zeros(B, cap, 2, device="cuda")
+            cache = (first[0].clone(), first[1].clone(), zero, zero)
+            outs.append(run_gpu(qw, c, st, cache, wide[:, pad:], starts, T, 1.0e7, hd // 4, out_dtype=tdt, max_len=cap))
+            flags.append(c.device_error())
+            torch.cuda.synchronize()
+            caches.append(cache)
+            c.close()
+        assert flags[0] == flags[1] and (flags[0] != 0) == any(s + T > cap for s in starts)
+        assert torch.equal(caches[0][0], caches[1][0]) and torch.equal(caches[0][1], caches[1][1])
+        err = relerr(host(outs[0]), host(outs[1]))
+        print("f32 shares", B, T, cap, hd, pad, err)
+        assert err <= (2e-5 if io == "f32" else 8e-3), err
