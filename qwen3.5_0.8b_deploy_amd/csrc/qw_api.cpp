@@ -942,11 +942,14 @@ static qw_status run_gemm(qw_ctx* ctx, const qw_weight* W, int rows, const void*
     // occupy at least half the CUs: the prefill shapes, and from a few hundred
     // tokens on the wide projections (measured at 520 / 1024 tokens: gate/up
     // 30.7 / 28.3 -> 23.0 / 23.6 us, QKV+Z 34.3 -> 25.6 us at 520, Q+gate+K+V
-    // 30.8 -> 24.2 us at 1024).  Fewer blocks keep the 64-row split-K GEMM: a
-    // split-K direct-A kernel measured 1.7-2.9x slower on the 1024-row
-    // projections (its last workgroup reads every partial tile through one CU)
+    // 30.8 -> 24.2 us at 1024; INT8 gate/up 28.5 -> 25.0 at 520, 30.7 -> 26.3
+    // at 1000, 85.8 -> 71.7 at 4000).  INT8 with K >= 2048 needs more than half:
+    // at exactly half one wave per SIMD converts and multiplies in turn, and two
+    // K splits are faster (4000 x 3584 -> 1024: 69.8 -> 39.5 + 12.0 us)
+    const int da_blocks = (W->phys_tiles * 16 + 255) / 256 * ((M + 127) / 128);
+    const bool i8_deep = W->wf == QW_WFMT_INT8_ROWSCALE && W->K >= 2048;
     if (ctx->gemm_da && (rows == 256 || rows == 64) && !ctx->gemm_tile_m &&
-        (ctx->gemm_da == 2 || 2 * ((W->phys_tiles * 16 + 255) / 256 * ((M + 127) / 128)) >= ctx->num_cus) &&
+        (ctx->gemm_da == 2 || 2 * da_blocks >= ctx->num_cus + (i8_deep ? 1 : 0)) &&
         qwk::gemm_da_fits(a, W->wf, (int)xdt, ids != nullptr)) {
         a.group_m = ctx->gemm_da_group;
         const int nwv = ctx->gemm_da_waves
@@ -964,25 +967,32 @@ static qw_status run_gemm(qw_ctx* ctx, const qw_weight* W, int rows, const void*
     // k-steps, the partials within the workspace): at 1024 tokens 128-224
     // workgroups measured best (down 46.8 -> 24 us, out 34.0 -> 20.5 us; 448
     // workgroups 30.5 us), at 3072 tokens S = 2 (down 94 -> 40 us, out 61 ->
-    // 30 us).  QW_GEMM_DA_SPLIT forces S (0: off)
-    const int da_blocks = (W->phys_tiles * 16 + 255) / 256 * ((M + 127) / 128);
+    // 30 us).  INT8 takes the most splits that stay within one workgroup per CU
+    // instead (down at 1000 tokens: 7 splits 17.6 + 7.0 us, 4 splits 21.3 + 5.5;
+    // at 2000: 4 splits 25.4 + 9.1, 2 splits 35.1 + 7.0; past one per CU slower,
+    // at 700: 14 splits 16.3 + 8.8, 7 splits 15.9 + 5.6), and only from K = 2048
+    // on: gate/up (K = 1024) at 390 tokens is 19.5 + 6.9 us split, 24.0 in the
+    // LDS-staged GEMM.  QW_GEMM_DA_SPLIT forces S (0: off)
     if (ctx->gemm_da && ctx->gemm_da_split != 0 && (rows == 256 || rows == 64) && !ctx->gemm_tile_m && !ids &&
-        (ctx->gemm_da_split > 0 || 2 * da_blocks < ctx->num_cus)) {
+        (ctx->gemm_da_split > 0 || (W->wf == QW_WFMT_INT8_ROWSCALE ? i8_deep && 2 * da_blocks <= ctx->num_cus
+                                                                  : 2 * da_blocks < ctx->num_cus))) {
         qwk::GemmArgs d = a;
         d.splitk = 1;
         d.group_m = ctx->gemm_da_group;
         d.partials = reinterpret_cast<float*>(ctx->partials);
         int S = 0;
         if (qwk::gemm_da_fits(d, W->wf, (int)xdt, false)) {
+            const int k32 = W->K / 32;
             for (int sc = 2; sc <= 32; ++sc) {
-                if (W->ksteps % (4 * sc) != 0 || W->ksteps / sc < 8) continue;
+                if (k32 % (4 * sc) != 0 || k32 / sc < 8) continue;
                 if (qwk::gemm_da_split_bytes(d, sc) > ctx->partials_bytes) break;
                 if (ctx->gemm_da_split > 0) {
                     if (sc == ctx->gemm_da_split) S = sc;
                     continue;
                 }
+                if (i8_deep && 2 * da_blocks * S >= ctx->num_cus && da_blocks * sc > ctx->num_cus) break;
                 S = sc;
-                if (2 * da_blocks * sc >= ctx->num_cus) break;
+                if (!i8_deep && 2 * da_blocks * sc >= ctx->num_cus) break;
             }
         }
         if (S >= 2) {

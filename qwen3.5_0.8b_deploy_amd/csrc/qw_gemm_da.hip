@@ -1,5 +1,5 @@
-// qw_gemm_da.hip -- the prefill GEMM for BF16 weights and BF16 activations
-// at many tokens ("direct-A"):  y[m][n] = sum_k W[n][k] * x[m][k] (+ epilogue).
+// qw_gemm_da.hip -- the prefill GEMM for BF16 weights and BF16 activations,
+// or INT8 weights and F16 activations, at many tokens ("direct-A"):  y[m][n] = sum_k W[n][k] * x[m][k] (+ epilogue).
 //
 // Shape.  A workgroup of 4 waves computes 256 weight rows x 128 tokens; wave
 // w owns rows 64w..64w+63 for all 128 tokens (4 x 8 blocks of the 16x16x32
@@ -42,6 +42,20 @@
 // piece, sums the S partials in split order and runs the same epilogue
 // per element.  One workgroup reducing a whole block would read S x 128 KB
 // through one CU, which measured slower than not splitting.
+//
+// INT8 weights (per-row scales, F16 activations).  A 1 KB unit is 16 rows x
+// 64 k, lane l = r + 16g holding row r's k 16g..16g+15: its two halves,
+// converted exactly to f16 in registers, are the A operands of two 16x16x32
+// f16 MFMAs whose k slots 8g.. are the k 16g + 8s.. (s = 0, 1), so the B
+// fragment of step s is chunk 2g + s of the token's 128-byte line instead of
+// 4s + g.  The ring holds units (half the bytes and registers per k-step); a
+// k-step's 40 conversions run beside its 32 MFMAs.  The row scale multiplies
+// the accumulators once, before the epilogue or the partial store.  Against the
+// LDS-staged GEMM (qw_gemm.hip), which converts every weight fragment in each
+// of the waves that share it: gate/up 30.7 -> 26.3 us at 1000 tokens and 352 ->
+// 266 us (0.90 PFLOP/s) at 16384, down 41.6 -> 24.6 (7 splits) and 175 -> 137.
+// Beside BF16 (23 us at 1000 tokens): the conversions, 40 per wave and k-step
+// beside 32 MFMAs, hide under the other wave's MFMAs only in part.
 //
 // Buffers.  The weight and activation buffer descriptors start at the
 // workgroup's first row / token and end at the operands' end, so rows past
@@ -159,9 +173,11 @@ __device__ __forceinline__ void da_epilogue(const GemmArgs& a, const f32x4 (&acc
 // XCD order), partial accumulators out, no epilogue.
 // NWV waves (4, or 8 with line loads): 64 * NWV weight rows per block, the
 // activation stages shared by all of them.
-template <bool GLU, bool LINE, bool PART, int NWV = 4>
+template <bool GLU, bool LINE, bool PART, int NWV = 4, int WF = WF_BF16>
 __global__ __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) void gemm_da_kernel(GemmArgs a) {
     static_assert(NWV == 4 || (NWV == 8 && LINE && !PART), "8 waves: line loads, no split");
+    static_assert(WF == WF_BF16 || (WF == WF_I8 && LINE), "INT8: line loads");
+    constexpr bool I8 = WF == WF_I8;
     constexpr int QN = 16 / NWV;  // activation units per wave and stage (line loads)
     using E = DaEpi<GLU>;
     constexpr int D = DA_D, NS = LINE ? DA_NS2 : DA_NS;
@@ -194,7 +210,8 @@ __global__ __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) void gemm_da_kernel(Gem
     for (int i = 0; i < 4; ++i) va[i] = (uint32_t)(((wave * 4 + i) * a.ksteps * 64 + lane) * 16);
     // k-steps past the end reload the last one (never used)
     auto kc = [&](int ks) { return __builtin_amdgcn_readfirstlane(min(ks, ks_n - 1)); };
-    u32x4 A[D][4], B[8];
+    constexpr int RING = I8 ? 2 : D;  // weight units in flight per row tile
+    u32x4 A[RING][4], B[8];
     f32x4 acc[4][8];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -205,15 +222,17 @@ __global__ __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) void gemm_da_kernel(Gem
 #pragma unroll
         for (int i = 0; i < 4; ++i) dst[i] = __builtin_amdgcn_raw_buffer_load_b128(wrs, va[i], so, 0);
     };
-    auto mfma_step = [&](int u, const uint8_t* stn, int noff0, int noff1) {
+    auto mfma_step = [&](const u32x4 (&Au)[4], const uint8_t* stn, int noff0, int noff1) {
         // column j's B is refilled (k-step ks+1) as soon as its MFMAs are issued
         __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, A[u][i]),
-                                                                   __builtin_bit_cast(bf16x8, B[j]), acc[i][j], 0, 0, 0);
+                if constexpr (I8)
+                    acc[i][j] = mfma_f16(__builtin_bit_cast(f16x8, Au[i]), __builtin_bit_cast(f16x8, B[j]), acc[i][j]);
+                else
+                    acc[i][j] = mfma_bf16(__builtin_bit_cast(bf16x8, Au[i]), __builtin_bit_cast(bf16x8, B[j]), acc[i][j]);
             B[j] = *reinterpret_cast<const u32x4*>(stn + j * (LINE ? 2 * DA_U2 : 1024) + (LINE ? noff0 : 0));
         }
 #if QW_DA_SCHED
@@ -262,7 +281,7 @@ __global__ __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) void gemm_da_kernel(Gem
                 __builtin_amdgcn_s_waitcnt(vm_wait(4 + 6 * (NS - 3)));
                 __syncthreads();
                 dma(ks + NS - 1);
-                mfma_step(u, lds + ((ks + 1) % NS) * STG + lane * 16, 0, 0);
+                mfma_step(A[u], lds + ((ks + 1) % NS) * STG + lane * 16, 0, 0);
                 loadA(A[u], ks + D);
             }
         }
@@ -284,46 +303,91 @@ __global__ __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) void gemm_da_kernel(Gem
         }
         auto dma = [&](int p) {  // k-steps 2p, 2p+1
             uint8_t* st = lds + (p % NS) * STG + wave * QN * DA_U2;
-            const int so = kbase * 64 + __builtin_amdgcn_readfirstlane(min(p, (ks_n >> 1) - 1)) * 128;
+            const int so = I8 ? (kbase + kc(p)) * 128
+                              : kbase * 64 + __builtin_amdgcn_readfirstlane(min(p, (ks_n >> 1) - 1)) * 128;
 #pragma unroll
             for (int q = 0; q < QN; ++q) lds_dma16_so(xrs, st + q * DA_U2, vb[q], so);
         };
         const int t_rd = lane & 15, g_rd = lane >> 4;
         auto roff = [&](int s) {  // read offset of k-step parity s within a tile's pair of units
-            const int c = 4 * s + g_rd;
+            const int c = I8 ? 2 * g_rd + s : 4 * s + g_rd;
             return (t_rd >> 3) * DA_U2 + 16 * ((8 * c + ((t_rd & 7) ^ c)) ^ (8 * (t_rd >> 3)));
         };
         const int ro0 = roff(0), ro1 = roff(1);
 #pragma unroll
         for (int s0 = 0; s0 < NS; ++s0) dma(s0);
 #pragma unroll
-        for (int d = 0; d < D; ++d) loadA(A[d], d);
+        for (int d = 0; d < RING; ++d) loadA(A[d], d);
         __builtin_amdgcn_s_waitcnt(vm_wait(0));
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < 8; ++j) B[j] = *reinterpret_cast<const u32x4*>(lds + j * 2 * DA_U2 + ro0);
-        for (int ks0 = 0; ks0 < ks_n; ks0 += D) {
+        if constexpr (I8) {  // ks_n, kbase: in units of 64 k
+            for (int p0 = 0; p0 < ks_n; p0 += RING) {
 #pragma unroll
-            for (int u = 0; u < D; ++u) {
-                const int ks = ks0 + u;
-                const int p = ks >> 1;
-                if (u & 1) {
-                    // second k-step of pair p: our loads of pair p+1 have
-                    // landed (after them: 4 weight loads, QN + 8 loads per
-                    // later pair, 4 of this pair's first k-step), publish;
-                    // pair p's stage is free for pair p+NS
-                    __builtin_amdgcn_s_waitcnt(vm_wait(8 + (QN + 8) * (NS - 2)));
+                for (int u = 0; u < RING; ++u) {
+                    const int p = p0 + u;
+                    u32x4 F[4];
+                    auto half = [&](int w) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            uint32_t l, h;
+                            i8x4_to_f16(A[u][i][w], l, h);
+                            F[i][0] = l, F[i][1] = h;
+                            i8x4_to_f16(A[u][i][w + 1], l, h);
+                            F[i][2] = l, F[i][3] = h;
+                        }
+                    };
+                    half(0);
+                    mfma_step(F, lds + (p % NS) * STG, ro1, 0);
+                    half(2);
+                    // our loads of pair p+1 have landed (after them: QN + 4
+                    // loads per later pair), publish; pair p's stage is free
+                    // for pair p+NS.  The weight loads go first: the next
+                    // pair's conversions wait for all but the newest 4 loads,
+                    // which then are these activations (the other way round
+                    // 28.5 and 22.9 us for 26.6 and 21.1)
+                    __builtin_amdgcn_s_waitcnt(vm_wait((QN + 4) * (NS - 2)));
                     __syncthreads();
+                    loadA(A[u], p + RING);
                     dma(p + NS);
-                    mfma_step(u, lds + ((p + 1) % NS) * STG, ro0, 0);
-                } else {
-                    mfma_step(u, lds + (p % NS) * STG, ro1, 0);
+                    mfma_step(F, lds + ((p + 1) % NS) * STG, ro0, 0);
                 }
-                loadA(A[u], ks + D);
+            }
+        } else {
+            for (int ks0 = 0; ks0 < ks_n; ks0 += D) {
+#pragma unroll
+                for (int u = 0; u < D; ++u) {
+                    const int ks = ks0 + u;
+                    const int p = ks >> 1;
+                    if (u & 1) {
+                        // second k-step of pair p: our loads of pair p+1 have
+                        // landed (after them: 4 weight loads, QN + 8 loads per
+                        // later pair, 4 of this pair's first k-step), publish;
+                        // pair p's stage is free for pair p+NS
+                        __builtin_amdgcn_s_waitcnt(vm_wait(8 + (QN + 8) * (NS - 2)));
+                        __syncthreads();
+                        dma(p + NS);
+                        mfma_step(A[u], lds + ((p + 1) % NS) * STG, ro0, 0);
+                    } else {
+                        mfma_step(A[u], lds + (p % NS) * STG, ro1, 0);
+                    }
+                    loadA(A[u], ks + D);
+                }
             }
         }
     }
 
+    if constexpr (I8) {
+        const __amdgpu_buffer_rsrc_t srs = make_rsrc(a.scales, (uint32_t)a.n_tiles * 64u);  // rows past the end: 0
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const f32x4 sc = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                srs, ((nt0 + wave * 4 + i) * 16 + 4 * (lane >> 4)) * 4, 0, 0));
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc[i][j] = acc[i][j] * sc;
+        }
+    }
     if constexpr (PART) {
         // partial pieces [block][split][piece i*8+j][thread]
         f32x4* pp = reinterpret_cast<f32x4*>(a.partials) + ((size_t)b * S + sk) * 32 * 256 + threadIdx.x;
@@ -597,11 +661,11 @@ __global__ __launch_bounds__(256) void gemm_da_reduce(GemmArgs a) {
 
 bool gemm_da_fits(const GemmArgs& a, int wf, int xdt, bool argmax) {
     if (a.ldx % 8 != 0) return false;  // 16-byte activation chunks
-    if (wf != WF_BF16 || xdt != DT_BF16 || argmax || a.splitk > 1) return false;
+    if (!((wf == WF_BF16 && xdt == DT_BF16) || (wf == WF_I8 && xdt == DT_F16)) || argmax || a.splitk > 1) return false;
     if (a.N % 4 != 0 || !a.vec_store) return false;
     if ((a.flags & EP_SPLIT) && (a.split_period < 4 || (a.split_period & (a.split_period - 1)) != 0)) return false;
     if ((uint64_t)a.M * a.ldx * 2 >= (1ull << 31) || (uint64_t)a.n_tiles * a.ksteps * 1024 >= (1ull << 31)) return false;
-    return a.ksteps % DA_D == 0;
+    return a.ksteps % (wf == WF_I8 ? DA_D / 2 : DA_D) == 0;
 }
 
 size_t gemm_da_lds_bytes(bool glu, bool line, int nwv) {
@@ -609,6 +673,8 @@ size_t gemm_da_lds_bytes(bool glu, bool line, int nwv) {
 }
 
 hipError_t launch_gemm_da(const GemmArgs& a, bool glu, bool line, hipStream_t stream, int nwv, int persist_wgs) {
+    const bool i8 = a.scales != nullptr;
+    if (i8) line = true;
     if (nwv == 8 && !line) nwv = 4;
     GemmArgs b = a;
     const int rows = 64 * nwv;
@@ -616,7 +682,7 @@ hipError_t launch_gemm_da(const GemmArgs& a, bool glu, bool line, hipStream_t st
     b.nblk_m = (a.M + 127) / 128;
     int grid = b.nblk_n * b.nblk_m;
     const size_t lds = gemm_da_lds_bytes(glu, line, nwv);
-    if (nwv == 8 && persist_wgs >= 8) {
+    if (nwv == 8 && persist_wgs >= 8 && !i8) {
         // one workgroup per CU, a multiple of 8 (each XCD's share of the blocks)
         const int slots = std::min((grid + 7) / 8, persist_wgs / 8);
         auto kp = glu ? gemm_da_persist_kernel<true> : gemm_da_persist_kernel<false>;
@@ -634,6 +700,8 @@ hipError_t launch_gemm_da(const GemmArgs& a, bool glu, bool line, hipStream_t st
         hipLaunchKernelGGL(k, dim3(grid), dim3(64 * nwv), lds, stream, b);
         return hipGetLastError();
     };
+    if (i8 && nwv == 8) return glu ? go(gemm_da_kernel<true, true, false, 8, WF_I8>) : go(gemm_da_kernel<false, true, false, 8, WF_I8>);
+    if (i8) return glu ? go(gemm_da_kernel<true, true, false, 4, WF_I8>) : go(gemm_da_kernel<false, true, false, 4, WF_I8>);
     if (nwv == 8) return glu ? go(gemm_da_kernel<true, true, false, 8>) : go(gemm_da_kernel<false, true, false, 8>);
     if (line) return glu ? go(gemm_da_kernel<true, true, false>) : go(gemm_da_kernel<false, true, false>);
     return glu ? go(gemm_da_kernel<true, false, false>) : go(gemm_da_kernel<false, false, false>);
@@ -644,7 +712,9 @@ size_t gemm_da_split_bytes(const GemmArgs& a, int S) {
 }
 
 hipError_t launch_gemm_da_split(const GemmArgs& a, bool glu, bool line, int S, hipStream_t stream) {
-    if (S < 2 || a.ksteps % (DA_D * S) != 0 || !a.partials) return hipErrorInvalidValue;
+    const bool i8 = a.scales != nullptr;
+    if (i8) line = true;
+    if (S < 2 || a.ksteps % ((i8 ? DA_D / 2 : DA_D) * S) != 0 || !a.partials) return hipErrorInvalidValue;
     GemmArgs b = a;
     b.nblk_n = (a.n_tiles * 16 + 255) / 256;
     b.nblk_m = (a.M + 127) / 128;
@@ -659,7 +729,8 @@ hipError_t launch_gemm_da_split(const GemmArgs& a, bool glu, bool line, int S, h
         hipLaunchKernelGGL(k, dim3(blocks * S), dim3(256), lds, stream, b);
         return hipGetLastError();
     };
-    hipError_t e = line ? (glu ? go(gemm_da_kernel<true, true, true>) : go(gemm_da_kernel<false, true, true>))
+    hipError_t e = i8 ? (glu ? go(gemm_da_kernel<true, true, true, 4, WF_I8>) : go(gemm_da_kernel<false, true, true, 4, WF_I8>))
+                 : line ? (glu ? go(gemm_da_kernel<true, true, true>) : go(gemm_da_kernel<false, true, true>))
                         : (glu ? go(gemm_da_kernel<true, false, true>) : go(gemm_da_kernel<false, false, true>));
     if (e != hipSuccess) return e;
     if (glu) hipLaunchKernelGGL(gemm_da_reduce<true>, dim3(blocks * 16), dim3(256), 0, stream, b);
