@@ -89,7 +89,8 @@ struct qw_ctx {
     int attn_vcoal = -1;         // INT8 decode V loads: -1 by launch size, 0 scattered, 1 coalesced (QW_ATTN_VCOAL)
     bool attn_fused = true;      // one-launch INT8 decode attention (QW_ATTN_FUSED=0: prep / split / combine)
     int attn_prefill_min = 16;   // tokens per sequence from which the query-block attention kernel runs (QW_ATTN_PREFILL_MIN)  // tokens per sequence from which the chunked GDN form runs (QW_GDN_CHUNK_MIN)
-    int attn_pf_min = 32;  // QW_ATTN_PF_MIN: fewest tokens per sequence of the 32-token-block INT8 prefill
+    int attn_pf_min = 32;  // fewest tokens per sequence of the 64-token-block INT8 prefill
+    bool attn_pf_forced = false;  // QW_ATTN_PF_MIN set: that kernel from its token count on, whatever the work
     uint8_t* ws = nullptr;
     size_t ws_bytes = 0;
     // carved regions
@@ -262,7 +263,7 @@ qw_status qw_init(qw_ctx** out, int device, size_t workspace_bytes) {
     if (const char* v = getenv("QW_ATTN_SPLIT")) c->attn_split = std::max(0, atoi(v)) / 64 * 64;
     if (const char* v = getenv("QW_ATTN_VCOAL")) c->attn_vcoal = atoi(v) != 0 ? 1 : 0;
     if (const char* v = getenv("QW_ATTN_PREFILL_MIN")) c->attn_prefill_min = std::max(1, atoi(v));
-    if (const char* v = getenv("QW_ATTN_PF_MIN")) c->attn_pf_min = std::max(1, atoi(v));
+    if (const char* v = getenv("QW_ATTN_PF_MIN")) c->attn_pf_min = std::max(1, atoi(v)), c->attn_pf_forced = true;
     if (const char* v = getenv("QW_GDN_CHUNK_MIN")) c->gdn_chunk_min = std::max(1, atoi(v));
     if (const char* v = getenv("QW_WIDE")) c->wide = atoi(v) != 0;
     if (const char* v = getenv("QW_WIDE_MIN")) c->wide_min = std::max(1, atoi(v));
@@ -1345,10 +1346,20 @@ qw_status qw_attn_forward(qw_ctx* ctx, const qw_attn_params* p, const qw_kv_cach
             a.blk = 16;
         }
         a.lim = cache->dtype == QW_I8 ? a.nsplit * a.split : len;
-        // INT8, longer runs: 32-token query blocks over the cache expanded to
+        // INT8, longer runs: 64-token query blocks over the cache expanded to
         // f16 MFMA operands once per segment (attn_pf), wherever the workspace
-        // holds the expanded keys and a segment of rows
-        if (cache->dtype == QW_I8 && tokens >= ctx->attn_pf_min) {
+        // holds the expanded keys and a segment of rows.  Its four launches cost
+        // ~43 us before the keys count, the 16-token-block kernel ~12 us plus
+        // 0.08 us per key of a split while its workgroups are one per CU: it is
+        // worth them from 288 keys x 16-token blocks per CU on (1 x 512 tokens
+        // after 500: 65 K, 54 us against 44; 1 x 777: 76 K, 53 against 70; 8 x 128
+        // after 500: 80 K, 57 against 58; 3 x 256 after 500: 73 K, 55 against 45;
+        // 8 x 512: 512 K, 95 against 157), and where the eighth of the keys that
+        // one split walks is long (1 x 64 after 2000: 58 against 40; after 8000:
+        // 88 against 94; after 30000: 125 against 303)
+        const bool pf_pays = ctx->attn_pf_forced || a.split >= 832 ||
+                             (int64_t)batch * nkv * ((tokens + 15) / 16) * len >= (int64_t)288 * ctx->num_cus;
+        if (cache->dtype == QW_I8 && tokens >= ctx->attn_pf_min && pf_pays) {
             const int64_t keys = (std::min<int64_t>(cache->capacity, a.lim) + 63) / 64 * 64;
             const size_t kvb = (size_t)nkv * keys * qwk::attn_pf_bytes_per_key(hd);
             const size_t row = (size_t)nh * hd * 2, piece = qwk::attn_pf_bytes_per_piece(nh / nkv, hd);

@@ -12,16 +12,19 @@
 //   o_h = softmax(q_h . K_g^T / sqrt(hd)) V_g over positions 0 .. pos (causal),
 //   g = h / (nh / nkv); out = o * sigmoid(gate)
 //
-// Three launches per segment of rows:
-//   attn_prep     one workgroup per row: norms, RoPE, cache write, the
-//                 normalized q to the workspace;
-//   attn_split    (key split, KV head, row): the query heads of one KV group
-//                 (one wave each) over one range of keys, online softmax,
-//                 32-key tiles of K and V dequantized into LDS once for the
-//                 whole group; a partial (o, max, sum) per split;
-//   attn_combine  (row, head): merges the splits, gate, output.
-// Splits are sized so that a step fills the chip: many for one long decode
-// row, one per row for a prefill.  A token whose position lies outside the
+// Launches per segment of rows:
+//   decode and short runs: attn_prep (norms, RoPE, cache write, normalized q to
+//     the workspace), one workgroup per (key split, KV head, row)
+//     (attn_decode_i8h on f16 MFMA, attn_split for an FP32 cache), attn_combine
+//     (merges the splits, gate, output); a small INT8 decode step is the one
+//     launch attn_decode_i8h<., true>;
+//   INT8 prefill: attn_prep_rows, attn_expand (the cached codes and scales to
+//     f16 MFMA operands), attn_pf (64-token query blocks, keys cut into runs of
+//     equal work), attn_pf_merge; attn_prefill_i8h serves 16..31 tokens and
+//     workspaces too small for the expanded keys;
+//   FP32 prefill: attn_prep, attn_prefill (16-token blocks, keys cut into shares
+//     where the blocks leave the chip idle), attn_combine.
+// A token whose position lies outside the
 // cache (or beyond the max_len the launch was sized for) writes nothing,
 // outputs zeros and raises the context's device error flag.
 #include "qw_stream.hpp"

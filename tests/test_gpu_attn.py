@@ -308,7 +308,7 @@ def test_attn_prefill_blocks(qw, oracle, relerr, hd, nh, nkv, B, T, starts, io, 
         for c, m in zip(first[2:], (1.0, vmul)):
             c.copy_(torch.rand(c.shape, generator=gen, device="cuda") * 0.02 * m + 0.001)
         outs, caches, flags = [], [], []
-        for env in ({}, {"QW_ATTN_PF_MIN": "1000000"}):
+        for env in ({"QW_ATTN_PF_MIN": "32"}, {"QW_ATTN_PF_MIN": "1000000"}):
             c = _ctx_with(qw, env)
             cache = tuple(x.clone() for x in first)
             outs.append(run_gpu(qw, c, st, cache, wide[:, pad:], starts, T, 1.0e7, hd // 4,
