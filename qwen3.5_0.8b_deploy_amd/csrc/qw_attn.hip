@@ -92,8 +92,15 @@ __device__ __forceinline__ float wave_max(float v) {
     return fmaxf(v, butterfly<1>(v));
 }
 
-// Rotation of a pair, the roundings spelled out: every kernel that writes cache
-// codes has to round them alike.
+// Sum of squares of a lane's elements and rotation of a pair, the roundings
+// spelled out: every kernel that writes cache codes has to round them alike.
+template <int E>
+__device__ __forceinline__ float sum_squares(const float (&x)[E]) {
+    float ss = __builtin_fmaf(x[0], x[0], x[1] * x[1]);
+#pragma unroll
+    for (int e = 2; e < E; ++e) ss = __builtin_fmaf(x[e], x[e], ss);
+    return ss;
+}
 __device__ __forceinline__ float rope0(float x0, float x1, float c, float s) { return __builtin_fmaf(x0, c, -(x1 * s)); }
 __device__ __forceinline__ float rope1(float x0, float x1, float c, float s) { return __builtin_fmaf(x1, c, x0 * s); }
 
@@ -130,10 +137,7 @@ __global__ __launch_bounds__(1024) void attn_prep(AttnArgs a) {
 #pragma unroll
         for (int e = 0; e < E; ++e) x[e] = at_load(src, a.in_dt, base + e);
         if (isq || isk) {
-            float ss = 0.0f;
-#pragma unroll
-            for (int e = 0; e < E; ++e) ss = __builtin_fmaf(x[e], x[e], ss);
-            ss = wave_sum(ss);
+            const float ss = wave_sum(sum_squares(x));
             const float rms = sqrtf(ss / (float)HD + 1e-6f);
             const float* w = isq ? a.qn_w : a.kn_w;
 #pragma unroll
@@ -234,10 +238,7 @@ __global__ __launch_bounds__(1024) void attn_prep_rows(AttnArgs a) {
             if (i >= nr) break;
             const int rl = blockIdx.x * R + i;
             if (isq || isk) {
-                float ss = 0.0f;
-#pragma unroll
-                for (int e = 0; e < E; ++e) ss = __builtin_fmaf(x[i][e], x[i][e], ss);
-                ss = wave_sum(ss);
+                const float ss = wave_sum(sum_squares(x[i]));
                 const float rms = sqrtf(ss / (float)HD + 1e-6f);
                 const float* w = isq ? a.qn_w : a.kn_w;
 #pragma unroll
@@ -1706,10 +1707,7 @@ __global__ __launch_bounds__(256) void attn_decode_i8h(AttnArgs a) {
 #pragma unroll
             for (int e = 0; e < E; ++e) x[e] = at_load(src, a.in_dt, base + e);
             if (it <= G) {  // q or k: RMSNorm (1 + w), then RoPE on d < rot
-                float ss = 0.0f;
-#pragma unroll
-                for (int e = 0; e < E; ++e) ss = __builtin_fmaf(x[e], x[e], ss);
-                ss = wave_sum(ss);
+                const float ss = wave_sum(sum_squares(x));
                 const float rms = sqrtf(ss / (float)HD + 1e-6f);
                 const float* w = isq ? a.qn_w : a.kn_w;
 #pragma unroll

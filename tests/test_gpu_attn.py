@@ -358,3 +358,38 @@ def test_attn_prefill_f32_shares(qw, oracle, relerr, B, T, cap, starts, hd, io):
         err = relerr(host(outs[0]), host(outs[1]))
         print("f32 shares", B, T, cap, hd, pad, err)
         assert err <= (2e-5 if io == "f32" else 8e-3), err
+
+
+@pytest.mark.parametrize("int8,T,hd", [(False, 1, 256), (True, 1, 256), (True, 40, 256), (True, 20, 128), (True, 1, 128)])
+def test_attn_key_norm_rounding(qw, oracle, int8, T, hd):
+    """The keys' norm is summed in one order by every kernel that writes the
+    cache (the row kernel, its four-row form, the one-launch decode): per lane
+    x1^2, then x0^2, x2^2, x3^2 fused onto it, then lanes 32, 16, .. 1 apart.
+    FP32 cache: the keys bit for bit; INT8: their scales.  The keys have 13
+    fraction bits, so that squares and partial sums are exact in double and
+    each step below rounds once."""
+    B, nkv, E = 96 // min(T, 4), 2, hd // 64
+    st = Stream(oracle, B, T, 2300 + hd, hd=hd)
+    rows = np.round(st.rows * 8192.0).astype(np.float32) / np.float32(8192.0)
+    c = _ctx_with(qw, {"QW_ATTN_PF_MIN": "32"})
+    cache = qw.kv_cache(B, T, nkv, hd, int8=int8)
+    run_gpu(qw, c, st, cache, dev(rows.reshape(B * T, -1)), [0] * B, T, 1.0e7, 0)
+    torch.cuda.synchronize()
+    c.close()
+    f32, f64 = np.float32, np.float64
+    k = rows[..., st.nh * 2 * hd:st.nh * 2 * hd + nkv * hd].reshape(B, T, nkv, hd)
+    x = k.reshape(B, T, nkv, 64, E)
+    sq = x.astype(f64) ** 2
+    ss = (sq[..., 0] + sq[..., 1].astype(f32)).astype(f32)
+    for e in range(2, E):
+        ss = (sq[..., e] + ss).astype(f32)
+    lane = np.arange(64)
+    for off in (32, 16, 8, 4, 2, 1):
+        ss = ss + ss[..., lane ^ off]
+    rms = np.sqrt(((ss[..., :1] / f32(hd)).astype(f64) + f64(f32(1e-6))).astype(f32))
+    y = k / rms * (f32(1.0) + st.kn)
+    if int8:
+        m = np.abs(y).max(axis=-1) / f32(127.0)
+        assert np.array_equal(host(cache[2]), m)
+    else:
+        assert np.array_equal(host(cache[0]), y)
