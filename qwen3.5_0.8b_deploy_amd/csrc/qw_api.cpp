@@ -1361,44 +1361,29 @@ qw_status qw_attn_forward(qw_ctx* ctx, const qw_attn_params* p, const qw_kv_cach
                              (int64_t)batch * nkv * ((tokens + 15) / 16) * len >= (int64_t)288 * ctx->num_cus;
         if (cache->dtype == QW_I8 && tokens >= ctx->attn_pf_min && pf_pays) {
             const int64_t keys = (std::min<int64_t>(cache->capacity, a.lim) + 63) / 64 * 64;
-            const size_t kvb = (size_t)nkv * keys * qwk::attn_pf_bytes_per_key(hd);
-            const size_t row = (size_t)nh * hd * 2, piece = qwk::attn_pf_bytes_per_piece(nh / nkv, hd);
-            int min_units = std::min(ctx->num_cus, 32);
-            // a segment of nb sequences x ntok tokens: its rows, keys and the shares of
-            // a plan for at least min_units CUs fit, and its tiles count in 31 bits
-            auto blocks = [&](int64_t n) { return (n + qwk::kPfBlock - 1) / qwk::kPfBlock; };
-            auto fits = [&](int64_t nb, int64_t ntok) {
-                return nb * (kvb + (size_t)ntok * row) + qwk::attn_pf_shares(min_units, nb * nkv * blocks(ntok)) * piece <= ws &&
-                       (double)nb * nkv * blocks(ntok) * (keys / 32 + 1) < 2147483648.0;
-            };
-            int64_t nb = 0, ntok = 0;
-            for (; ntok < 32 && min_units >= 4; min_units /= 8) {  // 32, then 4 CUs (small workspaces)
-                nb = std::min<int64_t>(batch, 65535), ntok = tokens;
-                while (nb > 1 && !fits(nb, ntok)) nb = (nb + 1) / 2;
-                while (ntok >= 32 && !fits(nb, ntok)) ntok = ntok / 2 / 32 * 32;
-            }
-            if (ntok >= 32 && keys <= (1 << 21)) {
-                for (int b0 = 0; b0 < batch; b0 += (int)nb)
-                    for (int tb = 0; tb < tokens; tb += (int)ntok) {
+            const qwk::PfCall pc{nh, nkv, hd, ctx->num_cus, batch, tokens, keys, ws};
+            const qwk::PfSegments ps = qwk::pf_segments(pc);
+            if (ps.ntok >= 32) {
+                uint8_t* w = reinterpret_cast<uint8_t*>(ctx->xnorm);
+                for (int b0 = 0; b0 < batch; b0 += (int)ps.nb)
+                    for (int tb = 0; tb < tokens; tb += (int)ps.ntok) {
                         a.b0 = b0;
-                        a.nb = (int)std::min<int64_t>(nb, batch - b0);
+                        a.nb = (int)std::min<int64_t>(ps.nb, batch - b0);
                         a.tb = tb;
-                        a.ntok = (int)std::min<int64_t>(ntok, tokens - tb);
+                        a.ntok = (int)std::min<int64_t>(ps.ntok, tokens - tb);
                         a.row0 = b0 * tokens + tb;
                         a.rows = a.nb * a.ntok;
+                        const qwk::PfSegment g = qwk::pf_segment(pc, ps.min_units, a.nb, a.ntok);
                         a.pf_keys = (int)keys;
-                        uint8_t* w = reinterpret_cast<uint8_t*>(ctx->xnorm) + (size_t)a.rows * row;
-                        const size_t kb = (size_t)a.nb * nkv * keys * hd * 2;
-                        a.kx = w;
-                        a.vx = w + kb;
-                        a.sx = reinterpret_cast<float*>(w + 2 * kb);
-                        a.part = a.sx + (size_t)a.nb * nkv * (keys / 32) * 128;
-                        const size_t left = ws - (size_t)a.rows * row - a.nb * kvb;
-                        const int64_t nblk = a.nb * nkv * blocks(a.ntok);
-                        a.pf_units = ctx->num_cus;
-                        while (a.pf_units > min_units && qwk::attn_pf_shares(a.pf_units, nblk) * piece > left) a.pf_units /= 2;
-                        a.pf_lone = nblk > a.pf_units || qwk::attn_pf_units(a.pf_units, nblk) * piece > left;
-                        a.pf_grid = (int)(qwk::attn_pf_units(a.pf_units, nblk) + nkv);
+                        a.kx = w + g.k_off;
+                        a.vx = w + g.v_off;
+                        a.sx = reinterpret_cast<float*>(w + g.s_off);
+                        a.part = reinterpret_cast<float*>(w + g.part_off);
+                        a.pf_units = g.units;
+                        a.pf_lone = g.lone;
+                        a.pf_pieces = g.pieces;
+                        a.pf_room = g.room;
+                        a.pf_grid = g.grid;
                         hipError_t e = qwk::launch_attn(a, stream);
                         if (e != hipSuccess) return hip_fail(ctx, e, "attn launch");
                     }

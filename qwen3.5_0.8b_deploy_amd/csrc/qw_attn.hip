@@ -1075,32 +1075,11 @@ __global__ __launch_bounds__(256) void attn_prefill_i8h(AttnArgs a) {
 // Measured, INT8 cache, one sequence, 4096 tokens from position 0: attn_pf 104,
 // prep 27.6, expand 5.9, merge 25.4 us (the 16-token kernels: 759, 40, -, 43); the
 // whole call 811 -> 160 us.  777 tokens: 24 + 11 + 5 + 13 us.
-constexpr int PF_Q = 64;      // tokens per query block
-constexpr int PF_KT = 32;     // keys per tile
-constexpr int PF_SC = 128;    // floats per tile of scales: 32 K | 32 V | raise threshold | padding
-constexpr int PF_MIN = 4;     // fewest tiles per unit
-
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ uint32_t pf_uni(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 
-// The query blocks of one sequence, longest first: block j (tokens 64 (nblk - 1
-// - j) ..) has tiles(j) key tiles (up to two more than its last query needs).
-// The host bounds the segment's total tiles below 2^31.
-struct PfSeq {
-    uint32_t nblk, c, tmax;
-    __device__ __forceinline__ PfSeq(const AttnArgs& a, int P0) {
-        const int pend = min(a.cap, a.lim);
-        nblk = (a.ntok + PF_Q - 1) / PF_Q;
-        tmax = (uint32_t)(pend + PF_KT - 1) / PF_KT;
-        c = (uint32_t)(min(max(P0, 0), pend) + a.tb + PF_KT - 1) / PF_KT;
-    }
-    __device__ __forceinline__ uint32_t tiles(uint32_t j) const { return min(c + 2 * (nblk - j), tmax); }
-    __device__ __forceinline__ uint32_t all() const {  // sum over the blocks, c + 2, c + 4, .. clamped to tmax
-        const uint32_t k = tmax > c ? min((tmax - c) / 2, nblk) : 0u;  // blocks below the clamp
-        return k * c + k * (k + 1) + (nblk - k) * tmax;
-    }
-};
+__device__ __forceinline__ PfSeq pf_seq(const AttnArgs& a, int P0) { return PfSeq(min(a.cap, a.lim), a.tb, a.ntok, P0); }
 
 __device__ __forceinline__ uint32_t pf_sum(uint32_t v) {
 #pragma unroll
@@ -1111,14 +1090,8 @@ __device__ __forceinline__ uint32_t pf_sum(uint32_t v) {
 // Longest unit, in tiles, of the segment's plan.  All lanes take part.
 __device__ __forceinline__ uint32_t pf_longest(const AttnArgs& a) {
     uint32_t v = 0;
-    for (int i = threadIdx.x & 63; i < a.nb; i += 64) v += PfSeq(a, a.pos[a.b0 + i]).all();
-    const uint32_t total = pf_sum(v) * a.nkv;
-    const uint32_t k = total / a.pf_units;
-    return max((uint32_t)PF_MIN, k + k * 3 / 10 + 2);
-}
-
-__device__ __forceinline__ uint32_t pf_shares(const PfSeq& q, uint32_t ut, uint32_t j) {
-    return max((q.tiles(j) + ut - 1) / ut, 1u);
+    for (int i = threadIdx.x & 63; i < a.nb; i += 64) v += pf_seq(a, a.pos[a.b0 + i]).all();
+    return pf_unit_tiles(pf_sum(v) * a.nkv, a.pf_units);
 }
 
 // Whether a block's units leave partials
@@ -1163,7 +1136,7 @@ __device__ __forceinline__ int pf_seq_of(const AttnArgs& a, uint32_t ut, uint32_
         for (int i0 = 0; i0 < a.nb; i0 += 64) {
             units = cut = 0;
             if (i0 + lane < a.nb) {
-                const PfSeq q(a, a.pos[a.b0 + i0 + lane]);
+                const PfSeq q = pf_seq(a, a.pos[a.b0 + i0 + lane]);
                 pf_count<false>(a, q, ut, q.nblk, units, cut);
             }
             uint32_t iu = units, ic = cut;
@@ -1182,7 +1155,7 @@ __device__ __forceinline__ int pf_seq_of(const AttnArgs& a, uint32_t ut, uint32_
     }
     int bl = 0;
     for (; bl < a.nb; ++bl) {
-        const PfSeq q(a, __builtin_amdgcn_readfirstlane(a.pos[a.b0 + bl]));
+        const PfSeq q = pf_seq(a, __builtin_amdgcn_readfirstlane(a.pos[a.b0 + bl]));
         pf_count<true>(a, q, ut, q.nblk, units, cut);
         if (u < units) break;
         u -= units;
@@ -1271,7 +1244,7 @@ __global__ __launch_bounds__(512, 2) void attn_pf(AttnArgs a) {
     const int bl = pf_seq_of(a, ut, u, slot);
     if (bl >= a.nb) return;  // uniform
     const int P0 = __builtin_amdgcn_readfirstlane(a.pos[a.b0 + bl]);
-    const PfSeq sq(a, P0);
+    const PfSeq sq = pf_seq(a, P0);
     uint32_t jb = 0, n = 0;  // block in unit order, its units; u: the share
     for (uint32_t j0 = 0; j0 < sq.nblk; j0 += 64) {
         const uint32_t v = j0 + lane < sq.nblk ? pf_shares(sq, ut, j0 + lane) : 0u, k = pf_cut(a, v) ? v : 0u;
@@ -1290,6 +1263,12 @@ __global__ __launch_bounds__(512, 2) void attn_pf(AttnArgs a) {
         slot += pf_uni(__shfl(ic, 63));
     }
     if (n == 0) return;  // past the last unit; uniform
+    // The grid's last workgroup of a head lies past every plan, and the partials
+    // hold every plan's (pf_most_units, pf_most_shares): flagged if that were not so
+    if ((int)blockIdx.x >= a.pf_room || (pf_cut(a, n) && (int)slot * a.nkv + g >= a.pf_pieces)) {
+        if (threadIdx.x == 0) *a.err = 1u;
+        return;
+    }
     const int qb = (int)(sq.nblk - 1 - jb);
     const int pend = min(a.cap, a.lim);
     const int b = a.b0 + bl, h = g * G + w, tok0 = a.tb + qb * PF_Q + 32 * tg;
@@ -1518,23 +1497,27 @@ __global__ __launch_bounds__(256) void attn_pf_merge(AttnArgs a) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int h = blockIdx.y / (PF_Q / 16), bl = blockIdx.z, G = a.nh / a.nkv, g = h / G, w = h % G;
     const uint32_t jb = blockIdx.x, ut = pf_longest(a);
-    const PfSeq sq(a, __builtin_amdgcn_readfirstlane(a.pos[a.b0 + bl]));
+    const PfSeq sq = pf_seq(a, __builtin_amdgcn_readfirstlane(a.pos[a.b0 + bl]));
     const int n = (int)pf_shares(sq, ut, jb);
     if (!pf_cut(a, n)) return;
     uint32_t slot = 0, units, cut;
     for (int i = threadIdx.x & 63; i < bl && (uint32_t)bl > sq.nblk; i += 64) {  // lanes take sequences
-        const PfSeq o(a, a.pos[a.b0 + i]);
+        const PfSeq o = pf_seq(a, a.pos[a.b0 + i]);
         pf_count<false>(a, o, ut, o.nblk, units, cut);
         slot += cut;
     }
     slot = pf_sum(slot);
     for (int i = 0; i < bl && (uint32_t)bl <= sq.nblk; ++i) {  // lanes take blocks
-        const PfSeq o(a, __builtin_amdgcn_readfirstlane(a.pos[a.b0 + i]));
+        const PfSeq o = pf_seq(a, __builtin_amdgcn_readfirstlane(a.pos[a.b0 + i]));
         pf_count<true>(a, o, ut, o.nblk, units, cut);
         slot += cut;
     }
     pf_count<true>(a, sq, ut, jb, units, cut);
     slot += cut;
+    if ((int)(slot + n - 1) * a.nkv + g >= a.pf_pieces) {  // never (as in attn_pf)
+        if (threadIdx.x == 0) *a.err = 1u;
+        return;
+    }
     const int qb = (int)(sq.nblk - 1 - jb), nq = min(PF_Q, a.ntok - qb * PF_Q);
     const int64_t ps = pf_piece(G, HD), next = ps * a.nkv;
     const float* p0 = a.part + ((int64_t)slot * a.nkv + g) * ps;
@@ -1952,9 +1935,6 @@ __global__ __launch_bounds__(256) void attn_decode_i8h(AttnArgs a) {
 size_t attn_bytes_per_row(int nh, int hd, int nsplit) {
     return (size_t)nh * hd * 4 + (size_t)nh * nsplit * (hd + 2) * 4;
 }
-
-size_t attn_pf_bytes_per_piece(int G, int hd) { return (size_t)G * PF_Q * (hd + 2) * 4; }
-size_t attn_pf_bytes_per_key(int hd) { return (size_t)2 * hd * 2 + PF_SC * 4 / PF_KT; }
 
 template <int HD>
 static void launch_combine(const AttnArgs& a, hipStream_t stream) {

@@ -1,10 +1,10 @@
 // qw_kernels.hpp -- host-visible launch descriptors of the gfx950 kernels.
 #pragma once
 
-#include <algorithm>
-
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include "qw_attn_plan.hpp"
 
 namespace qwk {
 
@@ -342,10 +342,12 @@ struct AttnArgs {
     int prefill;           // query-block kernel: tokens [tb, tb + ntok) of sequences [b0, b0 + nb)
     int b0, nb, tb, ntok;  // (the rows of the segment are then contiguous: row0 = b0*T + tb)
     unsigned* cnt;         // one-launch decode (T == 1, INT8): arrival counters [rows][nkv], zero between launches
-    // INT8 prefill of long token runs (attn_pf): the CUs its plan aims at (0: the
-    // 16-token kernels), its grid, keys per sequence of the expanded cache, and its
-    // buffers; qn then holds f16, part the shares' partials
-    int pf_units, pf_grid, pf_keys, pf_lone;  // pf_lone: uncut blocks write the output themselves
+    // INT8 prefill of long token runs (attn_pf, plan in qw_attn_plan.hpp): the CUs
+    // its plan aims at (0: the 16-token kernels), its grid and the workgroups of it
+    // that any plan fits into, keys per sequence of the expanded cache, partials that
+    // fit, and its buffers; qn then holds f16, part the shares' partials
+    int pf_units, pf_grid, pf_room, pf_keys, pf_pieces;
+    int pf_lone;           // uncut blocks write the output themselves
     uint8_t* kx;           // [nb][nkv][pf_keys][hd] f16, in MFMA operand order
     uint8_t* vx;
     float* sx;             // [nb][nkv][pf_keys / 32][128]: scales per 32-key tile
@@ -353,18 +355,6 @@ struct AttnArgs {
 };
 // workspace bytes per row for a given split count
 size_t attn_bytes_per_row(int nh, int hd, int nsplit);
-// attn_pf: bytes per key and KV head of the expanded cache (codes and scales),
-// and of one share's partial (G query heads per KV head).
-size_t attn_pf_bytes_per_key(int hd);
-size_t attn_pf_bytes_per_piece(int G, int hd);
-constexpr int kPfBlock = 64;  // tokens per query block
-// Most units of a plan for `units` CUs over `blocks` blocks (a block of t tiles
-// has at most t / ut + 1, ut >= 1.3 total / units), and most that belong to
-// blocks of more than one (at most 2 t / (ut + 1) each).
-inline int64_t attn_pf_units(int units, int64_t blocks) { return (int64_t)units * 10 / 13 + 1 + blocks; }
-inline int64_t attn_pf_shares(int units, int64_t blocks) {
-    return std::min((int64_t)units * 20 / 13 + 1, attn_pf_units(units, blocks));
-}
 hipError_t launch_attn(const AttnArgs& a, hipStream_t stream);
 
 // Token-embedding gather and the decode-step position advance (qw_embed.hip).

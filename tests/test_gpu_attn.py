@@ -324,6 +324,61 @@ def test_attn_prefill_blocks(qw, oracle, relerr, hd, nh, nkv, B, T, starts, io, 
         assert err <= (1e-3 if io == "f32" else 8e-3 if io == "bf16" else 2e-3), err
 
 
+def _random_cache(qw, B, cap, seed=3):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    cache = qw.kv_cache(B, cap)
+    for c in cache[:2]:
+        c.copy_(torch.randint(-127, 128, c.shape, generator=gen, device="cuda", dtype=torch.int8))
+    for c in cache[2:]:
+        c.copy_(torch.rand(c.shape, generator=gen, device="cuda") * 0.02 + 0.001)
+    return cache
+
+
+@pytest.mark.parametrize("B,T,cap,start,mb", [
+    (1, 64, 16384, 16250, 0),  # a block cut into 85 shares: the newest keys are its last one
+    (1, 128, 8192, 8000, 0),
+    (1, 192, 32768, 5280, 0),  # a cache much longer than the contexts
+    (4, 64, 4096, 3968, 0),
+    (1, 64, 32768, 0, 0),
+    # workspaces (MiB) that cut the call: a plan for 4 CUs, one sequence at a time;
+    # 2 sequences, then 1; 96 tokens of a sequence at a time; every unit a partial; a
+    # plan for 64 CUs
+    (3, 200, 1024, 700, 5), (3, 200, 1024, 800, 8), (3, 200, 1024, 824, 10), (3, 200, 1024, 0, 12),
+    (3, 200, 1024, 500, 32),
+])
+def test_attn_prefill_blocks_plan(qw, oracle, relerr, B, T, cap, start, mb):
+    """Contexts where the plan of the 64-token blocks is tight (shares just below
+    the units its grid has room for) and workspaces that cut the call into
+    segments, against the 16-token kernels and, the last query of each sequence,
+    against the oracle's attention over the cache as written.  A first call over
+    NaN scales fills the workspace's partials, so that a share nobody computed
+    shows."""
+    st = Stream(oracle, B, T, 3100 + T)
+    rows = dev(st.rows.reshape(B * T, -1))
+    first = _random_cache(qw, B, cap)
+    kw = {"workspace_bytes": qw.lib().qw_workspace_query(1, 1, 1) + (mb << 20)} if mb else {}
+    outs = []
+    for env in ({"QW_ATTN_PF_MIN": "32"}, {"QW_ATTN_PF_MIN": "1000000"}):
+        c = _ctx_with(qw, env, **kw)
+        cache = tuple(x.clone() for x in first)
+        nan = (cache[0], cache[1], torch.full_like(cache[2], float("nan")), torch.full_like(cache[3], float("nan")))
+        run_gpu(qw, c, st, nan, rows, [start] * B, T, 1.0e7, ROT, max_len=cap)
+        cache = tuple(x.clone() for x in first)
+        outs.append(host(run_gpu(qw, c, st, cache, rows, [start] * B, T, 1.0e7, ROT, max_len=cap)))
+        assert c.device_error() == 0
+        c.close()
+    err = relerr(outs[0], outs[1])
+    print("plan", B, T, cap, start, mb, err)
+    assert err <= 1e-3, err  # as test_attn_prefill_blocks
+    P = start + T - 1
+    for b in range(B):
+        q, g, k, _ = st.parts(st.rows[b, T - 1:T])
+        qn, _ = oracle.attn_norm_rope(q[0], k[0], st.qn, st.kn, P, NH, NKV, HD, ROT, 1.0e7)
+        kc, vc = (host(cache[i][b, :P + 1]) * host(cache[i + 2][b, :P + 1])[..., None] for i in (0, 1))
+        ref = oracle.attn_token(qn, g[0], kc, vc, NH, NKV, HD)
+        assert relerr(outs[0].reshape(B, T, -1)[b, -1], ref) <= 5e-3, b
+
+
 @pytest.mark.parametrize("B,T,cap,starts,hd,io", [
     (1, 16, 600, [500], 256, "f32"),           # one block, its keys cut
     (1, 300, 1024, [700], 256, "f32"),         # up to the last cache slot
