@@ -1331,6 +1331,9 @@ qw_status qw_attn_forward(qw_ctx* ctx, const qw_attn_params* p, const qw_kv_cach
         // query blocks of 16 tokens; segments of whole sequences, or of 16-token
         // chunks of one sequence, whose normalized q fit the workspace
         a.prefill = 1;
+        auto row_bytes = [&](int nsplit) {
+            return (size_t)nh * hd * 4 + (nsplit > 1 ? (size_t)nh * nsplit * (hd + 2) * 4 : 0);
+        };
         if (cache->dtype == QW_I8) {
             // key splits of >= 256 keys, at most 8 per query block (the longest
             // block's chain is then <= 1/8 of the context)
@@ -1338,11 +1341,14 @@ qw_status qw_attn_forward(qw_ctx* ctx, const qw_attn_params* p, const qw_kv_cach
             a.split = std::max(256, (s8 + 31) / 32 * 32);
             a.nsplit = (len + a.split - 1) / a.split;
         } else {
-            // about 2.5 workgroups per CU, at most 8 shares of >= 128 keys
+            // about 2.5 workgroups per CU, at most 8 shares of >= 128 keys, and no
+            // more than the workspace holds for the whole call: where it has to be
+            // cut into segments, their rows come first
             const int64_t wgs = (int64_t)batch * nkv * ((tokens + 15) / 16);
             a.split = len;
             a.nsplit = (int)std::max<int64_t>(1, std::min<int64_t>({(int64_t)5 * ctx->num_cus / 2 / wgs, (int64_t)8,
                                                                     (int64_t)(len + 127) / 128}));
+            while (a.nsplit > 1 && (size_t)rows_all * row_bytes(a.nsplit) > ws) --a.nsplit;
             a.blk = 16;
         }
         a.lim = cache->dtype == QW_I8 ? a.nsplit * a.split : len;
@@ -1390,7 +1396,7 @@ qw_status qw_attn_forward(qw_ctx* ctx, const qw_attn_params* p, const qw_kv_cach
                 return QW_OK;
             }
         }
-        const size_t per_row = (size_t)nh * hd * 4 + (a.nsplit > 1 ? (size_t)nh * a.nsplit * (hd + 2) * 4 : 0);
+        const size_t per_row = row_bytes(a.nsplit);
         const int64_t seq_fit = (int64_t)(ws / (per_row * (size_t)tokens));
         if (seq_fit >= 1) {
             const int64_t nbseg = std::min<int64_t>({(int64_t)batch, seq_fit, (int64_t)65535});

@@ -415,6 +415,27 @@ def test_attn_prefill_f32_shares(qw, oracle, relerr, B, T, cap, starts, hd, io):
         assert err <= (2e-5 if io == "f32" else 8e-3), err
 
 
+@pytest.mark.parametrize("B,T", [(1, 16), (2, 40), (2, 150)])
+def test_attn_prefill_f32_smallest_workspace(qw, oracle, relerr, B, T):
+    """24 heads of 256 over an FP32 cache in the smallest workspace (3 MB): one row
+    of normalized q is 24 KB, with 8 key shares' partials 218 KB.  16 tokens fit
+    only with fewer shares, 2 x 40 with one, 2 x 150 with one and in segments of 128
+    tokens; against the default workspace (FP32 throughout, 2e-5)."""
+    nh, nkv, cap, start = 24, 6, 1100, 930
+    st = Stream(oracle, B, T, 2700 + T, nh=nh, nkv=nkv)
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    first = [torch.randn(B, cap, nkv, HD, generator=gen, device="cuda") for _ in range(2)]
+    outs = []
+    for kw in ({}, {"workspace_bytes": 1}):
+        c = _ctx_with(qw, {}, **kw)
+        zero = torch.zeros(B, cap, nkv, device="cuda")
+        cache = (first[0].clone(), first[1].clone(), zero, zero)
+        outs.append(host(run_gpu(qw, c, st, cache, dev(st.rows.reshape(B * T, -1)), [start] * B, T, 1.0e7, ROT)))
+        assert c.device_error() == 0
+        c.close()
+    assert relerr(outs[1], outs[0]) <= 2e-5
+
+
 @pytest.mark.parametrize("int8,T,hd", [(False, 1, 256), (True, 1, 256), (True, 40, 256), (True, 20, 128), (True, 1, 128)])
 def test_attn_key_norm_rounding(qw, oracle, int8, T, hd):
     """The keys' norm is summed in one order by every kernel that writes the
