@@ -415,6 +415,27 @@ def test_attn_prefill_f32_shares(qw, oracle, relerr, B, T, cap, starts, hd, io):
         assert err <= (2e-5 if io == "f32" else 8e-3), err
 
 
+@pytest.mark.parametrize("int8,hd,io", [(True, 256, "f32"), (True, 256, "bf16"), (True, 256, "f16"), (True, 128, "f32"),
+                                        (False, 256, "bf16")])
+def test_attn_prefill_lone_split_rows(qw, ctx, oracle, relerr, int8, hd, io):
+    """16-token blocks whose keys are one split write the output themselves, four
+    dims per access or, for rows at an odd column, by elements: the same values
+    (1e-6, the same FP32 steps; 16-bit outputs equal), and the oracle's."""
+    B, T, cap = 2, 61, 64
+    st = Stream(oracle, B, T, 2500 + hd, hd=hd)
+    tdt = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}[io]
+    rows = dev(st.rows.reshape(B * T, -1)).to(tdt)
+    outs = []
+    for pad in (0, 1):
+        wide = torch.zeros(B * T, st.ld + 4, device="cuda", dtype=tdt)
+        wide[:, pad:pad + st.ld] = rows
+        cache = qw.kv_cache(B, cap, st.nkv, hd, int8=int8)
+        outs.append(host(run_gpu(qw, ctx, st, cache, wide[:, pad:], [0, 3], T, 1.0e7, hd // 4, out_dtype=tdt)))
+    assert relerr(outs[0], outs[1]) <= (1e-6 if io == "f32" else 0.0)
+    ref, _ = oracle_stream(oracle, st, host(rows).reshape(B, T, -1)[0], int8, 1.0e7, hd // 4, cap)
+    assert relerr(outs[0].reshape(B, T, -1)[0], ref) <= (5e-3 if io == "f32" else 1e-2)
+
+
 @pytest.mark.parametrize("B,T", [(1, 16), (2, 40), (2, 150)])
 def test_attn_prefill_f32_smallest_workspace(qw, oracle, relerr, B, T):
     """24 heads of 256 over an FP32 cache in the smallest workspace (3 MB): one row
