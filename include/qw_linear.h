@@ -314,7 +314,8 @@ qw_status qw_device_error(qw_ctx* ctx, int* flag);
  * interleaved Q|gate projection output with gate = q + 256, 256 for split
  * buffers); k and v at r*ld_in + g*head_dim + d.  positions: device int
  * [batch].  max_len: an upper bound of positions[b] + tokens used to size the
- * launch (0: the cache capacity).  A token whose position falls outside the
+ * launch (0: the cache capacity); the nearer it is, the better the kernels fit
+ * the call.  A token whose position falls outside the
  * cache writes nothing, outputs zeros and sets the device error flag
  * (qw_device_error).  head_dim 128 or 256, num_heads / num_kv_heads <= 4. */
 typedef struct {

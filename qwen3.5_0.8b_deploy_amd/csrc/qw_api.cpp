@@ -1354,22 +1354,12 @@ qw_status qw_attn_forward(qw_ctx* ctx, const qw_attn_params* p, const qw_kv_cach
         a.lim = cache->dtype == QW_I8 ? a.nsplit * a.split : len;
         // INT8, longer runs: 64-token query blocks over the cache expanded to
         // f16 MFMA operands once per segment (attn_pf), wherever the workspace
-        // holds the expanded keys and a segment of rows.  Its four launches cost
-        // ~43 us before the keys count, the 16-token-block kernel ~12 us plus
-        // 0.08 us per key of a split while its workgroups are one per CU: it is
-        // worth them from 288 keys x 16-token blocks per CU on (1 x 512 tokens
-        // after 500: 65 K, 54 us against 44; 1 x 777: 76 K, 53 against 70; 8 x 128
-        // after 500: 80 K, 57 against 58; 3 x 256 after 500: 73 K, 55 against 45;
-        // 8 x 512: 512 K, 95 against 157), and where the eighth of the keys that
-        // one split walks is long (1 x 64 after 2000: 58 against 40; after 8000:
-        // 88 against 94; after 30000: 125 against 303)
-        const bool pf_pays = ctx->attn_pf_forced || a.split >= 832 ||
-                             (int64_t)batch * nkv * ((tokens + 15) / 16) * len >= (int64_t)288 * ctx->num_cus;
-        if (cache->dtype == QW_I8 && tokens >= ctx->attn_pf_min && pf_pays) {
+        // holds the expanded keys and a segment of rows, and that pays (pf_pays)
+        if (cache->dtype == QW_I8 && tokens >= ctx->attn_pf_min) {
             const int64_t keys = (std::min<int64_t>(cache->capacity, a.lim) + 63) / 64 * 64;
             const qwk::PfCall pc{nh, nkv, hd, ctx->num_cus, batch, tokens, keys, ws};
             const qwk::PfSegments ps = qwk::pf_segments(pc);
-            if (ps.ntok >= 32) {
+            if (ps.ntok >= 32 && (ctx->attn_pf_forced || qwk::pf_pays(pc, ps, len, max_len > 0, a.split, a.nsplit))) {
                 uint8_t* w = reinterpret_cast<uint8_t*>(ctx->xnorm);
                 for (int b0 = 0; b0 < batch; b0 += (int)ps.nb)
                     for (int tb = 0; tb < tokens; tb += (int)ps.ntok) {

@@ -104,6 +104,44 @@ inline PfSegments pf_segments(const PfCall& p) {
     }
 }
 
+// Whether the segments' launches take less time than the 16-token-block kernel,
+// which cuts each block's keys into nsplit splits of `split`.  len: the keys per
+// sequence that the launch is sized for; known: that is the caller's bound of the
+// sequences' lengths, not just the cache's capacity.  Measured (us, 8 heads over 2
+// KV heads of 256, 256 CUs; the 64-token blocks against the 16-token ones):
+// - one split: the 16-token kernel writes the outputs itself, without a merge
+//   (64 x 96 tokens alone 114 : 93, 200 x 32 after 224 188 : 162, 64 x 160 182 : 179).
+// - Four launches per segment cost ~43 before the keys count, the other kernel ~12
+//   and 0.08 per key of a split while its workgroups are one per CU: worth it from
+//   288 keys x 16-token blocks per CU and segment (1 x 512 after 500: 65 K, 54 : 44;
+//   1 x 777: 76 K, 53 : 70; 8 x 128 after 500: 80 K, 57 : 58; 8 x 512: 512 K, 95 :
+//   157), and where one split is long (1 x 64 after 2000 58 : 40, after 8000 88 : 94,
+//   after 30000 125 : 303).
+// - Of a run of one or two blocks per sequence each expanded key is used little.
+//   Once the expanded keys outgrow the memory-side cache (from ~144 MB: 8 x 32 after
+//   8000 91 : 103, after 10500 175 : 122) fits of both sides decide: 30 per segment,
+//   0.8 per sequence and the expanded bytes at 1.15 TB/s, 0.6 times that again for a
+//   second block, against rounds of workgroups of 13 + 0.08 per key (8 x 32 after
+//   30000 535 : 308, 16 x 32 after 30000 1073 : 597, 16 x 80 1698 : 1480, 8 x 64 after 10000
+//   189 : 221, 3 x 32 after 28000 231 : 279; from 96 tokens on the blocks win, 8 x 96
+//   after 30000 850 : 900).
+// - Keys not known: only the run's own are certain, and the other kernel, its splits
+//   sized for the capacity, walks them in one: worth it from 72 keys x blocks per CU
+//   and segment (position 0, capacity 32768: 1 x 256 44 : 38, 1 x 400 49 : 73, 8 x 256
+//   in four segments 196 : 177, 8 x 100 180 : 62, 64 x 100 1465 : 412; capacity 2048: 64
+//   x 100 157 : 412), and not for a block that is half empty (100 x 32, 130 : 102).
+inline bool pf_pays(const PfCall& p, const PfSegments& s, int64_t len, bool known, int64_t split, int64_t nsplit) {
+    if (nsplit <= 1) return false;
+    const int64_t nseg = (p.batch + s.nb - 1) / s.nb * ((p.tokens + s.ntok - 1) / s.ntok);
+    const int64_t blocks = (int64_t)p.batch * p.nkv * ((p.tokens + 15) / 16);
+    if (!known) return p.tokens >= 48 && blocks * std::min<int64_t>(p.tokens, len) >= 72 * p.cus * nseg;
+    if (split < 832 && blocks * len < 288 * p.cus * nseg) return false;
+    const double bytes = (double)p.batch * p.seq_bytes();
+    if (p.tokens >= 96 || bytes <= 144e6) return true;
+    const double rounds = std::max(1.0, (double)blocks * nsplit / p.cus);
+    return 30.0 * nseg + 0.8 * p.batch + bytes * (p.tokens > PF_Q ? 1.6 : 1.0) / 1.15e6 < rounds * (13.0 + 0.08 * split);
+}
+
 // One segment's launch.  Workspace: rows of f16 queries | K | V | scales | partials.
 struct PfSegment {
     int units;    // CUs the plan aims at

@@ -60,7 +60,50 @@ static bool check_call(int nh, int nkv, int hd, int cus, size_t ws, int batch, i
     return true;
 }
 
+// the route of a call of 8 heads over 2 KV heads of 256 on 256 CUs, its splits cut
+// as qw_attn_forward cuts them
+static bool route(int batch, int tokens, int len, bool known, size_t ws = 180u << 20) {
+    const int split = std::max(256, ((len + 7) / 8 + 31) / 32 * 32), nsplit = (len + split - 1) / split;
+    const PfCall p{8, 2, 256, 256, batch, tokens, ((int64_t)len + 63) / 64 * 64, ws};
+    const PfSegments s = pf_segments(p);
+    return s.ntok >= 32 && pf_pays(p, s, len, known, split, nsplit);
+}
+
+// A cache's spare capacity takes no call to the 64-token blocks that its keys do not.
+static bool check_routes() {
+    struct R { int batch, tokens, len; bool known, blocks; };
+    std::vector<R> rs;
+    for (int cap : {4096, 8192, 32768})
+        for (const R& r : {R{1, 64, 0, false, false}, R{1, 144, 0, false, false}, R{1, 256, 0, false, false},
+                           R{8, 100, 0, false, false}, R{1, 777, 0, false, true}, R{1, 4096, 0, false, true}})
+            rs.push_back({r.batch, r.tokens, std::max(cap, r.tokens), false, r.blocks});
+    for (const R& r : {R{64, 100, 8192, false, false}, R{64, 100, 32768, false, false}, R{64, 100, 2048, false, true},
+                       R{100, 32, 1024, false, false}, R{1, 64, 64, true, false}, R{8, 100, 100, true, false},
+                       R{1, 64, 30064, true, true}, R{1, 512, 1012, true, false}, R{1, 777, 777, true, true},
+                       R{8, 512, 512, true, true}, R{16, 32, 30032, true, false}, R{8, 32, 8032, true, true},
+                       R{8, 32, 10532, true, false}, R{16, 80, 30080, true, false}, R{8, 64, 10064, true, true}, R{8, 100, 32100, true, true},
+                       R{1, 4096, 4096, true, true}})
+        rs.push_back(r);
+    for (const R& r : rs)
+        if (route(r.batch, r.tokens, r.len, r.known) != r.blocks) {
+            printf("violation: route of %d x %d, %d keys (%sknown): not the %d-token blocks\n", r.batch, r.tokens, r.len,
+                   r.known ? "" : "not ", r.blocks ? 64 : 16);
+            return false;
+        }
+    // a bound at its loosest makes no difference to calls whose keys are not known
+    for (int batch : {1, 2, 5, 8, 30, 64})
+        for (int tokens = 32; tokens <= 512; tokens += 16)
+            for (int len = 1024; len <= 65536; len *= 2)
+                if (route(batch, tokens, 2 * len, false) && !route(batch, tokens, len, false)) {
+                    printf("violation: %d x %d takes the 64-token blocks for a capacity of %d, not of %d\n", batch, tokens,
+                           2 * len, len);
+                    return false;
+                }
+    return true;
+}
+
 int main() {
+    if (!check_routes()) return 1;
     const size_t big = 180u << 20;
     // one sequence, and several at one position, at every position up to 32768:
     // a cache just long enough, and one of 32768

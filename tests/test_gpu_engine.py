@@ -321,3 +321,40 @@ def test_engine_check_raises_on_device_error(qw, ctx, oracle, relerr):
         ref = oracle.mlp_f64(oracle.round_bf16(G), oracle.round_bf16(U), oracle.round_bf16(D), host(x)) + host(x)
         assert relerr(host(y), ref) <= 2e-3
     assert ctx.device_error() == 0
+
+
+def test_engine_prefill_after_unseen_steps(qw, ctx, oracle, relerr):
+    """A prefill sizes its attention by the positions that the host has seen.
+    Steps replayed from a graph it does not see, a tensor handed out may change:
+    the same tokens as for the engine whose every step is seen (FP32 throughout,
+    other key shares: 1e-4), and no position beyond the launch."""
+    em = _engine_mod()
+    B, T, V, cap, steps = 2, 40, 1024, 1024, 6
+    layers = make_layers(oracle, 4, 7000)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    tl = [{k: dev(v) for k, v in L.items()} for L in layers]
+    fn, emb = dev(oracle.normal((em.H,), 6999, 0.0, 0.1)), dev(oracle.normal((V, em.H), 6998))
+    kw = dict(fmt=qw.WFMT_F32, lm_fmt=qw.WFMT_F32, kv_int8=False)
+    seen, graph, moved = (em.DecodeEngine(qw, ctx, tl, fn, emb, B, cap, **kw) for _ in range(3))
+    prompt = torch.from_numpy(np.random.default_rng(8).integers(0, V, (B, T)).astype(np.int32)).cuda()
+    stream = torch.cuda.Stream()
+    g = qw.Graph(ctx, stream)
+    with torch.cuda.stream(stream):
+        with g:
+            graph.step(stream=stream)
+    for e in (seen, graph, moved):
+        e.reset([3, 4])
+        e.prefill(prompt)
+    torch.cuda.synchronize()
+    for _ in range(steps):
+        seen.step()
+        moved.step()
+        g.launch(stream)
+        stream.synchronize()  # one context, one workspace
+    moved.pos.add_(cap - 2 * T - steps - 1)  # near the end of the cache, over keys of zero
+    for e in (seen, graph, moved):
+        e.prefill(prompt)  # raises if a position lies past the keys that the launch was sized for
+    assert seen._end == 2 * T + steps and graph._end is None and moved._end is None
+    assert torch.equal(seen.ids, graph.ids)
+    assert relerr(host(graph.x), host(seen.x).astype(np.float64)) <= 1e-4
+    assert moved.pos.tolist() == [cap - 1] * B
