@@ -118,13 +118,13 @@ inline PfSegments pf_segments(const PfCall& p) {
 //   157), and where one split is long (1 x 64 after 2000 58 : 40, after 8000 88 : 94,
 //   after 30000 125 : 303).
 // - Of a run of one or two blocks per sequence each expanded key is used little.
-//   Once the expanded keys outgrow the memory-side cache (from ~144 MB: 8 x 32 after
-//   8000 91 : 103, after 10500 175 : 122) fits of both sides decide: 30 per segment,
-//   0.8 per sequence and the expanded bytes at 1.15 TB/s, 0.6 times that again for a
-//   second block, against rounds of workgroups of 13 + 0.08 per key (8 x 32 after
-//   30000 535 : 308, 16 x 32 after 30000 1073 : 597, 16 x 80 1698 : 1480, 8 x 64 after 10000
-//   189 : 221, 3 x 32 after 28000 231 : 279; from 96 tokens on the blocks win, 8 x 96
-//   after 30000 850 : 900).
+//   For half a block over many keys, and once the expanded keys outgrow the
+//   memory-side cache (from ~144 MB), fits of both sides decide: 30 per segment, 0.8
+//   per sequence and the expanded bytes at 1.15 TB/s, 0.6 times that again for a
+//   second block, against rounds of workgroups of 13 + 0.08 per key (8 x 32 after 8000
+//   113 : 97, after 30000 535 : 308, 16 x 32 after 30000 1073 : 597, 16 x 80 1698 : 1480,
+//   8 x 64 after 10000 189 : 221, 3 x 32 after 28000 231 : 279, 4 x 32 after 14000 99 : 151;
+//   from 96 tokens on the blocks win, 8 x 96 after 30000 850 : 900).
 // - Keys not known: only the run's own are certain, and the other kernel, its splits
 //   sized for the capacity, walks them in one: worth it from 72 keys x blocks per CU
 //   and segment (position 0, capacity 32768: 1 x 256 44 : 38, 1 x 400 49 : 73, 8 x 256
@@ -137,7 +137,7 @@ inline bool pf_pays(const PfCall& p, const PfSegments& s, int64_t len, bool know
     if (!known) return p.tokens >= 48 && blocks * std::min<int64_t>(p.tokens, len) >= 72 * p.cus * nseg;
     if (split < 832 && blocks * len < 288 * p.cus * nseg) return false;
     const double bytes = (double)p.batch * p.seq_bytes();
-    if (p.tokens >= 96 || bytes <= 144e6) return true;
+    if (p.tokens >= 96 || (bytes <= 144e6 && (p.tokens > PF_Q / 2 || split < 832))) return true;
     const double rounds = std::max(1.0, (double)blocks * nsplit / p.cus);
     return 30.0 * nseg + 0.8 * p.batch + bytes * (p.tokens > PF_Q ? 1.6 : 1.0) / 1.15e6 < rounds * (13.0 + 0.08 * split);
 }
@@ -162,7 +162,10 @@ inline PfSegment pf_segment(const PfCall& p, int min_units, int64_t nb, int64_t 
     g.pieces = (int)std::min<size_t>((p.ws - g.part_off) / p.piece_bytes(), 1u << 30);
     const int64_t nblk = nb * p.nkv * p.blocks(ntok);
     g.units = p.cus;
-    while (g.units > min_units && pf_most_shares(g.units, nblk) > g.pieces) g.units /= 2;
+    // as many CUs as the partials allow, where the blocks alone do not fill the chip
+    // (8 x 100 tokens after 8000, room for 160: 367 us for 128 CUs, 266 for 165)
+    while (g.units > min_units && pf_most_shares(g.units, nblk) > g.pieces)
+        g.units -= nblk >= g.units ? (g.units + 1) / 2 : (g.units + 15) / 16;
     g.units = std::max(g.units, min_units);
     g.lone = nblk > g.units || pf_most_units(g.units, nblk) > g.pieces;
     g.room = (int)(pf_most_units(g.units, nblk) / p.nkv * p.nkv);

@@ -80,7 +80,7 @@ static bool check_routes() {
     for (const R& r : {R{64, 100, 8192, false, false}, R{64, 100, 32768, false, false}, R{64, 100, 2048, false, true},
                        R{100, 32, 1024, false, false}, R{1, 64, 64, true, false}, R{8, 100, 100, true, false},
                        R{1, 64, 30064, true, true}, R{1, 512, 1012, true, false}, R{1, 777, 777, true, true},
-                       R{8, 512, 512, true, true}, R{16, 32, 30032, true, false}, R{8, 32, 8032, true, true},
+                       R{8, 512, 512, true, true}, R{16, 32, 30032, true, false}, R{8, 32, 8032, true, false}, R{4, 32, 14032, true, true},
                        R{8, 32, 10532, true, false}, R{16, 80, 30080, true, false}, R{8, 64, 10064, true, true}, R{8, 100, 32100, true, true},
                        R{1, 4096, 4096, true, true}})
         rs.push_back(r);

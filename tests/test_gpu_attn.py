@@ -342,7 +342,7 @@ def _random_cache(qw, B, cap, seed=3):
     (1, 64, 32768, 0, 0),
     # workspaces (MiB) that cut the call: a plan for 4 CUs, one sequence at a time;
     # 2 sequences, then 1; 96 tokens of a sequence at a time; every unit a partial; a
-    # plan for 64 CUs
+    # plan for 86 CUs
     (3, 200, 1024, 700, 5), (3, 200, 1024, 800, 8), (3, 200, 1024, 824, 10), (3, 200, 1024, 0, 12),
     (3, 200, 1024, 500, 32),
 ])
