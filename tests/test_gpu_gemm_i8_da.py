@@ -4,6 +4,9 @@ accumulators) in its 4-wave, 8-wave and split-K forms, against FP64 on the
 stored codes, scales and F16 activations and against the LDS-staged INT8 GEMM
 (QW_GEMM_DA=0), plus bit-identical repeats.
 
+The GLU rows' split runs where their blocks are fewer than half the CUs (1040 rows
+of 520 here); 3584 make half a block per CU and more and are never split.
+
 Sizes: ragged token blocks (1, 127, 129 past a block), ragged row blocks
 (1008 = 63 tiles, 520), K = 1024 / 2048 / 3584 (8..28 rounds of the two-unit
 ring) and K = 128 (one round).  Bars: codes are exact in f16, products of f16
@@ -83,18 +86,24 @@ def test_i8_direct_a_residual(qw, ctx_f, oracle, relerr, N, K, M, form):
     assert relerr(host(outs[0]), host(outs[2]).astype(np.float64)) <= 1e-5
 
 
-@pytest.mark.parametrize("I,M,form", [(3584, 600, "w4"), (3584, 513, "w8"), (520, 200, "w4"), (3584, 520, "s2")])
+@pytest.mark.parametrize("I,M,form", [(3584, 600, "w4"), (3584, 513, "w8"), (520, 200, "w4"), (3584, 520, "s2"), (520, 200, "s2"),
+                                      (520, 129, "s2")])
 def test_i8_direct_a_glu(qw, ctx_f, oracle, relerr, I, M, form):
     H = 1024
     G = oracle.normal((I, H), 8130, 0.0, 0.02)
     U = oracle.normal((I, H), 8131, 0.0, 0.02)
     xt = dev(oracle.normal((M, H), 8133 + M), torch.float16)
-    ctx = ctx_f(form)
-    w = qw.Weight.pack_glu(ctx, G, U, qw.WFMT_INT8)
-    h = torch.empty(M, I, device="cuda")
-    qw.linear(ctx, w, xt, h)
-    torch.cuda.synchronize()
-    assert ctx.device_error() == 0
+    def run(form):
+        ctx = ctx_f(form)
+        w = qw.Weight.pack_glu(ctx, G, U, qw.WFMT_INT8)
+        h = torch.empty(M, I, device="cuda")
+        qw.linear(ctx, w, xt, h)
+        torch.cuda.synchronize()
+        assert ctx.device_error() == 0
+        return h
+    h = run(form)
+    if form == "s2":  # two sums of half the terms round otherwise than one: whether the split ran
+        assert torch.equal(h, run("w4")) == (I == 3584)
     xs = host(xt).astype(np.float64)
     g, u = xs @ codes(oracle, G).T, xs @ codes(oracle, U).T
     assert relerr(host(h), g / (1.0 + np.exp(-g)) * u) <= 1e-4
