@@ -678,7 +678,9 @@ __global__ __launch_bounds__(256, 2) void attn_prefill(AttnArgs a) {
     constexpr int ROW = HD + 4;                // LDS row stride, floats (bank spread)
     constexpr int PER = AT_KT * HD / 4 / 256;  // 16-byte chunks of a K (or V) tile per thread
     constexpr int KB = HD / 16, DT = HD / 16;
-    const int qb = blockIdx.x / a.nsplit, sp = blockIdx.x % a.nsplit, g = blockIdx.y, b = a.b0 + blockIdx.z;
+    // shares outermost: those that short sequences do not have come last, and the
+    // first ones spread over all XCDs (workgroup ids mod 8)
+    const int qb = blockIdx.x, sp = blockIdx.z / a.nb, g = blockIdx.y, b = a.b0 + blockIdx.z % a.nb;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
     const int G = a.nh / a.nkv;
     const int h = g * G + min(wave, G - 1);
@@ -1960,7 +1962,8 @@ static hipError_t launch_attn_hd(const AttnArgs& a, hipStream_t stream) {
                                stream, a);
             launch_combine<HD>(a, stream);
         } else {
-            hipLaunchKernelGGL((attn_prefill<HD>), dim3((a.ntok + 15) / 16 * a.nsplit, a.nkv, a.nb), dim3(256), 0,
+            // (nsplit > 1 only where blocks are few, so nb * nsplit stays a valid grid)
+            hipLaunchKernelGGL((attn_prefill<HD>), dim3((a.ntok + 15) / 16, a.nkv, a.nb * a.nsplit), dim3(256), 0,
                                stream, a);
             launch_combine<HD>(a, stream);
         }
