@@ -189,10 +189,14 @@ __global__ __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) void gemm_da_kernel(Gem
 
     // XCD-aware order (consecutive ids go to different XCDs: give each XCD a
     // contiguous range; the splits of a block are consecutive in it), then
-    // the grouped raster
+    // the grouped raster.  A small split grid without an even share per XCD keeps
+    // the ids' order where the splits divide 8: an XCD then has one K range of few
+    // blocks' activations (8224 rows at 193 tokens, 132 workgroups, 2 splits: 20.1 us,
+    // contiguous 22.7; 6160 at 300, 150: 20.8, 23.2; but 8224 at 300, 198: 23.8, 22.9;
+    // 1040 at 1100, 180, 4 splits: 22.5, 20.7; 1024 x 3584 at 600, 140, 7: 20.4, 19.0)
     const int nwg = gridDim.x;
     int b = blockIdx.x;
-    b = xcd_run(b, nwg);
+    if (!PART || (nwg & 7) == 0 || nwg >= 160 || (8 % a.splitk) != 0) b = xcd_run(b, nwg);
     const int S = PART ? a.splitk : 1;
     const int sk = PART ? b % S : 0;
     if constexpr (PART) b /= S;
