@@ -946,16 +946,23 @@ static qw_status run_gemm(qw_ctx* ctx, const qw_weight* W, int rows, const void*
     // 30.8 -> 24.2 us at 1024; INT8 gate/up 28.5 -> 25.0 at 520, 30.7 -> 26.3
     // at 1000, 85.8 -> 71.7 at 4000).  INT8 with K >= 2048 needs more than half:
     // at exactly half one wave per SIMD converts and multiplies in turn, and two
-    // K splits are faster (4000 x 3584 -> 1024: 69.8 -> 39.5 + 12.0 us)
+    // K splits are faster (4000 x 3584 -> 1024: 69.8 -> 39.5 + 12.0 us), for smaller K the
+    // LDS-staged GEMM's 64-row blocks (4096 x 1024 at 900 tokens 25.1 : 23.6, 8192 at 450
+    // 25.0 : 23.6, K = 512 18.7 : 15.9, K = 1536 the same; its 256-row blocks are not, 2048
+    // rows at 2000 25.4 : 28.9)
     const int da_blocks = (W->phys_tiles * 16 + 255) / 256 * ((M + 127) / 128);
-    const bool i8_deep = W->wf == QW_WFMT_INT8_ROWSCALE && W->K >= 2048;
+    const bool i8 = W->wf == QW_WFMT_INT8_ROWSCALE, i8_deep = i8 && W->K >= 2048;
     if (ctx->gemm_da && (rows == 256 || rows == 64) && !ctx->gemm_tile_m &&
-        (ctx->gemm_da == 2 || 2 * da_blocks >= ctx->num_cus + (i8_deep ? 1 : 0)) &&
+        (ctx->gemm_da == 2 || 2 * da_blocks >= ctx->num_cus + (i8_deep || (i8 && rows == 64) ? 1 : 0)) &&
         qwk::gemm_da_fits(a, W->wf, (int)xdt, ids != nullptr)) {
         a.group_m = ctx->gemm_da_group;
-        const int nwv = ctx->gemm_da_waves
-                            ? ctx->gemm_da_waves
-                            : ((W->phys_tiles * 16 + 511) / 512 * ((M + 127) / 128) >= ctx->num_cus ? 8 : 4);
+        const int nb8 = (W->phys_tiles * 16 + 511) / 512 * ((M + 127) / 128);  // blocks of 8 waves
+        // INT8: 8 waves only where their last round of one per CU is 5/8 full (6160 x
+        // 1024 rows at 2500 tokens, 260 blocks: 65 us, 4 waves 39, the LDS-staged GEMM
+        // 58; at 5000, 520: 98, 73, 90; 7168 at 4096, 448: 67, 68, 82)
+        const int last = (nb8 - 1) % ctx->num_cus + 1;
+        const bool tail = i8 && 8 * last < 5 * ctx->num_cus;
+        const int nwv = ctx->gemm_da_waves ? ctx->gemm_da_waves : (nb8 >= ctx->num_cus && !tail ? 8 : 4);
         hipError_t e = qwk::launch_gemm_da(a, W->glu != 0, ctx->gemm_da_line, stream, nwv,
                                            ctx->gemm_da_persist ? ctx->num_cus : 0);
         if (e != hipSuccess) return hip_fail(ctx, e, "gemm launch");

@@ -86,6 +86,21 @@ def test_i8_direct_a_residual(qw, ctx_f, oracle, relerr, N, K, M, form):
     assert relerr(host(outs[0]), host(outs[2]).astype(np.float64)) <= 1e-5
 
 
+@pytest.mark.parametrize("N,M", [(6160, 2500), (4096, 4096), (4096, 900)])
+def test_i8_route_by_rounds(qw, ctx, oracle, relerr, N, M):
+    """The unforced route where the 8-wave blocks' last round is nearly empty (260
+    blocks), where it is full (256), and at exactly half a block per CU, against FP64."""
+    K = 128
+    W = oracle.normal((N, K), 8150 + N, 0.0, 0.02)
+    xt = dev(oracle.normal((M, K), 8151 + M), torch.float16)
+    w = qw.Weight.pack(ctx, W, qw.WFMT_INT8)
+    y = torch.empty(M, N, device="cuda")
+    qw.linear(ctx, w, xt, y)
+    torch.cuda.synchronize()
+    assert ctx.device_error() == 0
+    assert relerr(host(y), host(xt).astype(np.float64) @ codes(oracle, W).T) <= 2e-5
+
+
 @pytest.mark.parametrize("I,M,form", [(3584, 600, "w4"), (3584, 513, "w8"), (520, 200, "w4"), (3584, 520, "s2"), (520, 200, "s2"),
                                       (520, 129, "s2")])
 def test_i8_direct_a_glu(qw, ctx_f, oracle, relerr, I, M, form):
