@@ -20,8 +20,9 @@
 //     launch attn_decode_i8h<., true>;
 //   INT8 prefill: attn_prep_rows, attn_expand (the cached codes and scales to
 //     f16 MFMA operands), attn_pf (64-token query blocks, keys cut into runs of
-//     equal work), attn_pf_merge; attn_prefill_i8h serves 16..31 tokens and
-//     workspaces too small for the expanded keys;
+//     equal work), attn_pf_merge; calls that do not pay for these four launches
+//     (pf_pays) or whose expanded keys the workspace does not hold: attn_prep,
+//     attn_prefill_i8h (16-token blocks), attn_combine;
 //   FP32 prefill: attn_prep, attn_prefill (16-token blocks, keys cut into shares
 //     where the blocks leave the chip idle), attn_combine.
 // A token whose position lies outside the
@@ -521,14 +522,14 @@ __device__ __forceinline__ void gate_store(const AttnArgs& a, int r, int h, int 
     }
 }
 
-// DC > 1 (many splits): blockIdx.z takes HD/DC of the head's dims, so more
-// workgroups share the split partials' reads (each recomputes M and l from
-// the splits' two floats).
 // Keys per share of a query block with L keys (the FP32 query-block kernel).
 __device__ __forceinline__ int block_share(const AttnArgs& a, int L) {
     return max(128, ((L + a.nsplit - 1) / a.nsplit + AT_KT - 1) / AT_KT * AT_KT);
 }
 
+// DC > 1 (many splits): blockIdx.z takes HD/DC of the head's dims, so more
+// workgroups share the split partials' reads (each recomputes M and l from
+// the splits' two floats).
 template <int HD, int NW, int DC = 1>
 __global__ __launch_bounds__(64 * NW) void attn_combine(AttnArgs a) {
     static_assert(DC == 1 || NW > 1, "dim chunks with the multi-wave merge");
@@ -669,9 +670,9 @@ __device__ __forceinline__ void tile_gate_store(const AttnArgs& a, const f32x4 (
 // group, each under the other's product.
 // Bound: the FP32 matrix cores (256 MFMAs of 32 cycles per wave and tile).  A
 // block's keys are cut into up to a.nsplit equal shares (at least 128 keys; the
-// number is chosen for about 2.5 workgroups per CU), merged by attn_combine:
-// without, 2 x 600 tokens make 152 workgroups, one per CU and the longest alone
-// at the end (317 -> 135 us, and 15 for the merge; without the cut 25.6 -> 15.7 us
+// number is chosen for about 2.5 workgroups per CU, two of which are resident),
+// merged by attn_combine: without, 2 x 600 tokens make 152 workgroups, one per CU and
+// the longest alone at the end (317 -> 138 us, and 15 for the merge; without the cut 25.6 -> 15.7 us
 // at 8 x 21 tokens, from the V rows spread over the LDS banks and 16-byte gates).
 template <int HD>
 __global__ __launch_bounds__(256, 2) void attn_prefill(AttnArgs a) {
@@ -1074,9 +1075,10 @@ __global__ __launch_bounds__(256) void attn_prefill_i8h(AttnArgs a) {
 // 128-register accumulator unscaled for nearly all tiles.  It is kept a whole
 // number (log2), so that neither it nor the cut into units changes the f16
 // rounding of the probabilities (down to f16's subnormals).
-// Measured, INT8 cache, one sequence, 4096 tokens from position 0: attn_pf 104,
-// prep 27.6, expand 5.9, merge 25.4 us (the 16-token kernels: 759, 40, -, 43); the
-// whole call 811 -> 160 us.  777 tokens: 24 + 11 + 5 + 13 us.
+// Measured, INT8 cache, one sequence, 4096 tokens from position 0: the call 809 ->
+// 159 us; in a kernel trace, which adds up to ~1 us to a launch, attn_pf 104, prep 28,
+// merge 26, expand 6 us (the 16-token kernels: 759, 40, 43, -).  777 tokens: 24 + 11 +
+// 13 + 5 us.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ uint32_t pf_uni(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
